@@ -1511,6 +1511,48 @@ def _awt_chunks(theta, lam, subgrid_size, margin, ub, vb):
     return uv_mid, corner
 
 
+# AW-towers sum groups directly up to this share of a visibility per pre-grid
+# cell ((2S)^2 cells per group): see aw_towers_imaging
+AWT_DIRECT_CELLS = 1024
+
+
+def _awt_bins_fft(rel, vt, gid, vstart_h, cstart_h, gwp, ga1, ga2, S, lam_sub, gcf, at, win,
+                  turns, lmag, max_stack_bytes):
+    """Chunk images [C, S, S] of AW-towers through pre-grids: batches of
+    groups of at most ``max_stack_bytes`` gridded onto [2S, 2S] each,
+    inverse transformed and summed per chunk."""
+    L, dev, M = _lib.load(), rel.device, 2 * S
+    Q, K = int(gcf.shape[0]), int(gcf.shape[1])
+    G, C = len(vstart_h) - 1, len(cstart_h) - 1
+    _lib.check(L.croc_awt_pregrid(_lib.ctx(), None, M, _lib.ptr(rel), 0, rel.shape[0],
+                                  float(lam_sub), Q, K, _lib.ptr(gcf), _lib.ptr(vt),
+                                  _lib.ptr(gid), 0, 1))
+    bins = torch.zeros((C, S, S), dtype=torch.complex64, device=dev)
+    gmax = max(1, int(max_stack_bytes) // (M * M * 8))
+    stack = torch.empty((min(G, gmax), M, M), dtype=torch.complex64, device=dev)
+    for g0 in range(0, G, gmax):
+        g1 = min(G, g0 + gmax)
+        sb = stack[:g1 - g0]
+        sb.zero_()
+        _lib.check(L.croc_awt_pregrid(_lib.ctx(), _lib.ptr(sb), M, _lib.ptr(rel),
+                                      int(vstart_h[g0]), int(vstart_h[g1]), float(lam_sub),
+                                      Q, K, _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(gid), g0, 0))
+        img = torch.fft.ifftn(sb, dim=(-2, -1), norm='forward')
+        c_lo = int(numpy.searchsorted(cstart_h, g0, side='right')) - 1
+        c_hi = int(numpy.searchsorted(cstart_h, g1, side='left'))
+        for c0 in range(c_lo, c_hi, 65535):
+            c1 = min(c_hi, c0 + 65535)
+            # group range of each chunk within the batch
+            starts = numpy.clip(cstart_h[c0:c1 + 1], g0, g1) - g0
+            st_t = torch.as_tensor(starts.astype(numpy.int32), device=dev)
+            _lib.check(L.croc_awt_apply(
+                _lib.ctx(), _lib.ptr(bins), c0, c1 - c0, _lib.ptr(img), S, _lib.ptr(st_t),
+                _lib.ptr(gwp[g0:g1]), _lib.ptr(ga1[g0:g1]), _lib.ptr(ga2[g0:g1]),
+                _lib.ptr(at), _lib.ptr(win), _lib.ptr(turns), _lib.ptr(lmag)))
+        del img
+    return bins
+
+
 def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa_gcf,
                       aa_subgrid, aa_subgrid2, aimage, wkern, dl=0.0, dm=0.0,
                       max_stack_bytes=4 << 30):
@@ -1595,47 +1637,39 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     vt = vc.to(torch.complex64).contiguous()
     lam_sub = S / theta
     L = _lib.load()
-    _lib.check(L.croc_awt_pregrid(_lib.ctx(), None, M, _lib.ptr(rel), 0, nv, float(lam_sub),
-                                  Q, K, _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(gid), 0, 1))
-    # image-space tables of the sub-grid
+    # image-space tables of the sub-grid; the window carries the inverse
+    # transform's 1 / M^2
     a2 = numpy.asarray(aa_subgrid2, dtype=float)[S // 2:S // 2 + S]
     a1 = numpy.asarray(aa_subgrid, dtype=float)
-    win = torch.as_tensor(numpy.outer(a1, a1) / numpy.outer(a2, a2), dtype=torch.float32,
-                          device=dev).contiguous()
-    wk = numpy.asarray(wkern.cpu().numpy() if _is_torch(wkern) else wkern, dtype=complex)
-    turns = torch.as_tensor(numpy.angle(wk) / (2 * numpy.pi), device=dev).contiguous()
-    lmag = torch.as_tensor(numpy.log2(numpy.abs(wk)), dtype=torch.float32,
-                           device=dev).contiguous()
+    win = torch.as_tensor(numpy.outer(a1, a1) / numpy.outer(a2, a2) / (M * M),
+                          dtype=torch.float32, device=dev).contiguous()
+    wk = _dev(wkern, torch.complex128)
+    turns = (torch.angle(wk) / (2 * math.pi)).contiguous()
+    lmag = torch.log2(torch.abs(wk)).to(torch.float32).contiguous()
     # group ranges: visibility offsets and chunk offsets
     vstart = torch.zeros(G + 1, dtype=torch.int64, device=dev)
     vstart[1:] = torch.cumsum(gcount, 0)
-    cstart = torch.zeros(C + 1, dtype=torch.int64, device=dev)
-    cstart[1:] = torch.cumsum(ccount, 0)
-    vstart_h, cstart_h = vstart.cpu().numpy(), cstart.cpu().numpy()
-    bins = torch.zeros((C, S, S), dtype=torch.complex64, device=dev)
+    cstart_h = numpy.concatenate([[0], numpy.cumsum(ccount.cpu().numpy())]).astype(numpy.int64)
     gwp32 = gwp.to(torch.int32).contiguous()
-    gmax = max(1, int(max_stack_bytes) // (M * M * 8))
-    stack = torch.empty((min(G, gmax), M, M), dtype=torch.complex64, device=dev)
-    for g0 in range(0, G, gmax):
-        g1 = min(G, g0 + gmax)
-        sb = stack[:g1 - g0]
-        sb.zero_()
-        _lib.check(L.croc_awt_pregrid(_lib.ctx(), _lib.ptr(sb), M, _lib.ptr(rel),
-                                      int(vstart_h[g0]), int(vstart_h[g1]), float(lam_sub),
-                                      Q, K, _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(gid), g0, 0))
-        img = torch.fft.ifftn(sb, dim=(-2, -1))
-        c_lo = int(numpy.searchsorted(cstart_h, g0, side='right')) - 1
-        c_hi = int(numpy.searchsorted(cstart_h, g1, side='left'))
-        for c0 in range(c_lo, c_hi, 65535):
-            c1 = min(c_hi, c0 + 65535)
-            # group range of each chunk within the batch
-            starts = numpy.clip(cstart_h[c0:c1 + 1], g0, g1) - g0
-            st_t = torch.as_tensor(starts.astype(numpy.int32), device=dev)
-            _lib.check(L.croc_awt_apply(
-                _lib.ctx(), _lib.ptr(bins), c0, c1 - c0, _lib.ptr(img), S, _lib.ptr(st_t),
-                _lib.ptr(gwp32[g0:g1]), _lib.ptr(ga1[g0:g1]), _lib.ptr(ga2[g0:g1]),
-                _lib.ptr(at), _lib.ptr(win), _lib.ptr(turns), _lib.ptr(lmag)))
-        del img
+    # Groups of few visibilities are summed directly (croc_awt_direct): ~15 ns
+    # per visibility, where the pre-grids cost ~1 us per (2S)^2 grid and
+    # 5 ns per visibility.  Measured with the awtowers1800 tracks repeated:
+    # S = 128, 1.8 visibilities per group 1.5 / 7.3 ms (direct / pre-grids),
+    # 32 times as many 7.3 / 9.1, 64 times 13.0 / 11.0; S = 64, 1.7 per group
+    # 1.4 / 2.7, 8 times 2.95 / 3.16, 16 times 4.7 / 3.7.  The line is one
+    # visibility per AWT_DIRECT_CELLS pre-grid cells.
+    if nv * AWT_DIRECT_CELLS <= G * M * M and M <= 4096:
+        bins = torch.empty((C, S, S), dtype=torch.complex64, device=dev)
+        vstart32 = vstart.to(torch.int32)
+        _lib.check(L.croc_awt_direct(
+            _lib.ctx(), _lib.ptr(bins), C, S, _lib.ptr(rel), nv, float(lam_sub), Q, K,
+            _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(vstart32),
+            cstart_h.ctypes.data_as(ctypes.c_void_p), _lib.ptr(gwp32), _lib.ptr(ga1),
+            _lib.ptr(ga2), _lib.ptr(at), _lib.ptr(win), _lib.ptr(turns), _lib.ptr(lmag),
+            min(int(max_stack_bytes), 1 << 30)))
+    else:
+        bins = _awt_bins_fft(rel, vt, gid, vstart.cpu().numpy(), cstart_h, gwp32, ga1, ga2, S,
+                             lam_sub, gcf, at, win, turns, lmag, max_stack_bytes)
     fb = torch.fft.fftn(bins, dim=(-2, -1))
     corner_t = torch.as_tensor(corner.astype(numpy.int32), device=dev).contiguous()
     for c0 in range(0, C, 65535):

@@ -249,6 +249,16 @@ int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
  * ([nant][S][S] cf32) times wkern^-gwp[g] (wkern = 2^lmag exp(2 pi i turns)
  * per pixel), all times win ([S][S]).
  *
+ * croc_awt_direct does the work of pregrid, inverse transform and apply in
+ * one step for groups of few visibilities: bins[c] ([nc][S][S] cf32,
+ * overwritten) = win times the sum over the chunk's groups g in [cstart[c],
+ * cstart[c + 1]) (cstart: host [nc + 1]) of S x S cut-out pixels of M^2
+ * times the inverse transform of the group's pre-grid (visibilities
+ * [vstart[g], vstart[g + 1]), vstart device [ngroups + 1]), each times the
+ * screen ratio and wkern^-gwp[g].  No empty groups or chunks; S <= 2048;
+ * at most max_bytes of partial sums.
+ * Same errors as the check_only croc_awt_pregrid, nothing written on them.
+ *
  * croc_awt_place adds (-1)^(x+y) bins[c] (forward transformed) into grid
  * ([N][N] cf32) at corner[c] = (x0, y0), clipped at the grid's edges. */
 int croc_awt_pregrid(croc_ctx *ctx, void *stack, int M, const double *rel, int64_t v0,
@@ -258,6 +268,12 @@ int croc_awt_apply(croc_ctx *ctx, void *bins, int c0, int nc, const void *stack,
                    const int32_t *start, const int32_t *gwp, const int32_t *ga1,
                    const int32_t *ga2, const void *ascreen, const float *win,
                    const double *turns, const float *lmag);
+int croc_awt_direct(croc_ctx *ctx, void *bins, int nc, int S, const double *rel,
+                    int64_t nv, double lam_sub, int Q, int K, const void *gcf,
+                    const void *vis, const int32_t *vstart, const int64_t *cstart,
+                    const int32_t *gwp, const int32_t *ga1, const int32_t *ga2,
+                    const void *ascreen, const float *win, const double *turns,
+                    const float *lmag, int64_t max_bytes);
 int croc_awt_place(croc_ctx *ctx, void *grid, int N, const void *bins, int nc, int S,
                    const int32_t *corner);
 

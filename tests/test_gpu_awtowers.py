@@ -95,3 +95,24 @@ def test_errors(gpu):
     empty = G.aw_towers_imaging(sc['theta'], sc['lam'], numpy.zeros((0, 3)),
                                 numpy.zeros((0, 2), dtype=int), numpy.zeros(0), *args[5:])
     assert empty.shape == (sc['N'], sc['N']) and not empty.any()
+
+
+@pytest.mark.parametrize('direct', [True, False])
+@pytest.mark.parametrize('S,margin,K,budget', [(32, 6, 6, 4 << 30),    # one pixel tile
+                                               (34, 8, 5, 4 << 30),    # ragged tiles, odd support
+                                               (64, 16, 7, 1),         # one segment per chunk
+                                               (96, 30, 8, 4 << 30)])
+def test_direct_and_transformed_groups(gpu, monkeypatch, direct, S, margin, K, budget):
+    """Group images summed directly (croc_awt_direct) and through pre-grids:
+    both against the oracle, for supports and sub-grids off the tile size and
+    chunks of one and of several segments."""
+    monkeypatch.setattr(G, 'AWT_DIRECT_CELLS', 0 if direct else 1 << 40)
+    print('case awtowers direct=%s S=%d K=%d' % (direct, S, K), flush=True)
+    sc = scenario(seed=5, S=S, margin=margin)
+    wk = R.w_kernel_function(sc['l'], sc['m'], 2.0)
+    gcf = R.kernel_oversample(sc['aa'], 64, K)
+    args = (sc['theta'], sc['lam'], sc['uvw'], sc['src'], sc['vis'], 2.0, S, margin, gcf,
+            sc['aa_sub'], sc['aa_sub2'], sc['aimage'], wk)
+    got = G.aw_towers_imaging(*args, max_stack_bytes=budget)
+    ref = AWT.aw_towers_imaging(*args)
+    assert rel(got, ref) < TOL, rel(got, ref)
