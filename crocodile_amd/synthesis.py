@@ -1354,11 +1354,11 @@ def _w_planes(uv, wstep):
     order: (plane numbers on the host, counts and mean w on the device)."""
     pl = torch.round(uv[:, 2] / float(wstep)).to(torch.int64)
     lo, hi = (int(x) for x in torch.stack([pl.min(), pl.max()]).cpu())
-    idx = pl - lo
-    counts = torch.bincount(idx, minlength=hi - lo + 1)
-    # per-block histograms: index_add_'s FP64 atomics onto a few dozen
-    # addresses serialise (half a second for 2e6 visibilities)
-    sums = torch.bincount(idx, weights=uv[:, 2], minlength=hi - lo + 1).to(torch.float64)
+    counts = torch.empty(hi - lo + 1, dtype=torch.int64, device=uv.device)
+    sums = torch.empty(hi - lo + 1, dtype=torch.float64, device=uv.device)
+    _lib.check(_lib.load().croc_wplane_sums(
+        _lib.ctx(), _lib.ptr(uv), uv.shape[0], uv.shape[1], float(wstep), lo, hi - lo + 1,
+        _lib.ptr(counts), _lib.ptr(sums)))
     nz = torch.nonzero(counts).reshape(-1)
     midw = sums[nz] / counts[nz].to(torch.float64)
     return pl, lo, hi - lo + 1, (nz + lo).cpu().tolist(), counts[nz], midw
@@ -1403,14 +1403,15 @@ def w_stacking_imaging(theta, lam, uvw, src, vis, wstep, max_stack_bytes=4 << 30
                                       uv.shape[0], uv.shape[1], float(lam), float(wstep),
                                       lo, ntab, _lib.ptr(slot_of), _lib.ptr(vt), centred))
         if centred:
-            img = torch.fft.ifftn(st, dim=(-2, -1))
+            img = torch.fft.ifftn(st, dim=(-2, -1), norm='forward')
         else:
             img = torch.fft.fftshift(torch.fft.ifftn(torch.fft.ifftshift(st, dim=(-2, -1)),
-                                                     dim=(-2, -1)), dim=(-2, -1))
+                                                     dim=(-2, -1), norm='forward'), dim=(-2, -1))
         mw = midw[b0:b0 + P].contiguous()
         _lib.check(L.croc_wstack_add(_lib.ctx(), _lib.ptr(image), _lib.ptr(img), P, N,
                                      float(theta), _lib.ptr(mw), centred))
         del img
+    image *= 1.0 / (N * N)  # the inverse transforms' scale, once on the sum
     return _out(image, like_torch)
 
 

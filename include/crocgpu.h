@@ -226,6 +226,12 @@ int croc_wstack_grid(croc_ctx *ctx, void *stack, int P, int N, const double *uvw
                      int64_t nv, int64_t stride, double lam, double wstep,
                      int64_t plane0, int ntab, const int32_t *slot_of, const void *vis,
                      int centred);
+/* croc_wplane_sums counts the visibilities of every w-plane t =
+ * round-half-even(w / wstep) - plane0, 0 <= t < ntab, and sums their w:
+ * count int64 [ntab], sum double [ntab] (overwritten; the planes' mean w of
+ * cell 10).  A plane outside the table is CROC_EPLANE. */
+int croc_wplane_sums(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride,
+                     double wstep, int64_t plane0, int ntab, int64_t *count, double *sum);
 int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
                     double theta, const double *midw, int centred);
 

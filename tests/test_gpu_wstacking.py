@@ -118,3 +118,34 @@ def test_errors_and_empty(gpu):
     assert not G.w_stacking_imaging(theta, lam, empty, None, numpy.zeros(0), 10.0).any()
     assert not G.w_stacking_subgrid_imaging(theta, lam, empty, None, numpy.zeros(0), 10.0,
                                             8).any()
+
+
+@pytest.mark.parametrize('ntab,nv,stride', [(1, 70_001, 3), (65, 70_001, 3), (4096, 5000, 4),
+                                            (4097, 5000, 3), (7, 1, 3)])
+def test_plane_sums(gpu, ntab, nv, stride):
+    """Counts and sums of w per plane, on both sides of the LDS table's size.
+    The sums' bound: nv roundings of at most eps/2 of the sum of |w|."""
+    from crocodile_amd import _lib
+    rng = numpy.random.default_rng(ntab)
+    wstep, plane0 = 2.5, -(ntab // 2)
+    uvw = numpy.zeros((nv, stride))
+    uvw[:, 2] = rng.uniform(plane0 - 0.49, plane0 + ntab - 0.51, nv) * wstep
+    uvw[0, 2] = (plane0 + 0.5) * wstep if ntab > 1 else 0.0   # a half-even tie
+    t = numpy.round(uvw[:, 2] / wstep).astype(int) - plane0
+    d = torch.as_tensor(uvw, device='cuda')
+    count = torch.full((ntab,), -1, dtype=torch.int64, device='cuda')
+    total = torch.full((ntab,), 7.0, dtype=torch.float64, device='cuda')
+    L = _lib.load()
+
+    def call(n):
+        return L.croc_wplane_sums(_lib.ctx(), _lib.ptr(d), nv, stride, wstep, plane0, n,
+                                  _lib.ptr(count), _lib.ptr(total))
+
+    _lib.check(call(ntab))
+    assert (count.cpu().numpy() == numpy.bincount(t, minlength=ntab)).all()
+    ref = numpy.bincount(t, weights=uvw[:, 2], minlength=ntab)
+    bound = nv * 2.0 ** -53 * numpy.abs(uvw[:, 2]).sum() + 1e-300
+    assert numpy.abs(total.cpu().numpy() - ref).max() <= bound
+    if ntab > 1 and t.max() == ntab - 1:
+        with pytest.raises(ValueError):
+            _lib.check(call(ntab - 1))
