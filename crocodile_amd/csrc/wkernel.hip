@@ -10,7 +10,8 @@
 //   ky = Q (y - S//2) + yf,  kx = Q (x - S//2) + xf,
 //
 // evaluated here as two dense passes (rows, then columns) with the twiddle
-// phase reduced exactly in integers before the FP64 sincospi.  The far field
+// phase reduced exactly in integers and looked up in a table of the F Q FP64
+// values (k_twiddles).  The far field
 // of a w-kernel, exp(2 pi i w (1 - sqrt(1 - l^2 - m^2))) on the coordinates
 // of kernel_coordinates (synthesis.py:250-293), is evaluated in FP64 on the
 // device, for all w-planes of a bank in one launch.
@@ -92,56 +93,113 @@ __global__ void k_wfarfield(FFArgs a, const double *__restrict__ w,
   ff[(int64_t)p * F * F + idx] = v;
 }
 
-// Row pass: tmp[p][m][kx] = sum_l ff[p][m][l] E(kx - Q(S//2), l), kx in [0, QS).
-__global__ void k_zoom_rows(const double2 *__restrict__ ff, int64_t ff_stride,
-                            int F, int Q, const int32_t *__restrict__ Sp,
-                            double2 *__restrict__ tmp, int64_t tmp_stride) {
-  const int p = blockIdx.y;
-  const int S = Sp[p];
-  const int QS = Q * S;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= F * QS) return;
-  const int m = idx / QS, kidx = idx - m * QS;
-  const int64_t k = (int64_t)kidx - (int64_t)Q * (S / 2);
-  const int64_t M = (int64_t)F * Q;
-  const double2 *row = ff + p * ff_stride + (int64_t)m * F;
-  double sr = 0.0, si = 0.0;
-  for (int l = 0; l < F; l++) {
-    const double2 t = twiddle(mod64(k * (l - F / 2), M), M);
-    const double2 f = row[l];
-    sr += f.x * t.x - f.y * t.y;
-    si += f.x * t.y + f.y * t.x;
-  }
-  tmp[p * tmp_stride + idx] = make_double2(sr, si);
+// tab[j] = exp(-2 pi i j / M), j in [0, M).
+__global__ void k_twiddles(int64_t M, double2 *__restrict__ tab) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < M) tab[j] = twiddle(j, M);
 }
 
-// Column pass and re-layout to [yf][xf][y][x].
-template <typename OutT>
-__global__ void k_zoom_cols(const double2 *__restrict__ tmp, int64_t tmp_stride,
-                            int F, int Q, const int32_t *__restrict__ Sp,
-                            const int64_t *__restrict__ out_off,
-                            OutT *__restrict__ out) {
-  const int p = blockIdx.y;
-  const int S = Sp[p];
-  const int QS = Q * S;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)QS * QS) return;
-  const int kyi = (int)(idx / QS), kxi = (int)(idx - (int64_t)kyi * QS);
-  const int64_t ky = (int64_t)kyi - (int64_t)Q * (S / 2);
-  const int64_t M = (int64_t)F * Q;
-  const double2 *col = tmp + p * tmp_stride + kxi;
-  double sr = 0.0, si = 0.0;
-  for (int m = 0; m < F; m++) {
-    const double2 t = twiddle(mod64(ky * (m - F / 2), M), M);
-    const double2 f = col[(int64_t)m * QS];
-    sr += f.x * t.x - f.y * t.y;
-    si += f.x * t.y + f.y * t.x;
+// The two passes are products of small dense complex FP64 matrices, bound by
+// the FP64 vector rate (78.6 TFLOP/s).  A lane takes one output column, a
+// wavefront ZOOM_R rows: the operand that depends on the row alone is
+// wave-uniform (scalar loads), the other is read once per lane and used
+// ZOOM_R times, so a term costs 4 FP64 instructions.  Columns are numbered
+// i = xf S + x (kx = Q x + xf), the order of the kernel tables, so
+// that both passes write runs of S elements.  101 planes, F = 64, Q = 8, S =
+// 15: 40 + 58 us (an FP64 sincospi per term took 235 + 347 us).
+constexpr int ZOOM_R = 8;
+constexpr int ZOOM_NT = 256;  // four wavefronts, 4 ZOOM_R rows
+
+__device__ __forceinline__ int zoom_wave_rows(int block) {
+  return (block * (ZOOM_NT / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) *
+         ZOOM_R;
+}
+
+// Row pass: tmp[p][m][i] = sum_l ff[p][m][l] E(k_i, l).
+__global__ __launch_bounds__(ZOOM_NT) void k_zoom_rows(
+    const double2 *__restrict__ ff, int64_t ff_stride, int F, int Q,
+    const int32_t *__restrict__ Sp, const double2 *__restrict__ tab, double2 *__restrict__ tmp,
+    int64_t tmp_stride) {
+  const int p = blockIdx.z;
+  const int S = Sp[p], QS = Q * S;
+  const uint32_t M = (uint32_t)F * (uint32_t)Q;  // below 2^31
+  const int m0 = zoom_wave_rows(blockIdx.y);
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (blockIdx.x * 64 >= QS || m0 >= F) return;
+  const int ii = min(i, QS - 1);
+  const int64_t k = (int64_t)Q * (ii % S - S / 2) + ii / S;
+  uint32_t idx = (uint32_t)mod64(-k * (F / 2), M);
+  const uint32_t step = (uint32_t)mod64(k, M);
+  const double2 *row[ZOOM_R];
+#pragma unroll
+  for (int r = 0; r < ZOOM_R; r++) row[r] = ff + p * ff_stride + (int64_t)min(m0 + r, F - 1) * F;
+  double sr[ZOOM_R], si[ZOOM_R];
+#pragma unroll
+  for (int r = 0; r < ZOOM_R; r++) sr[r] = si[r] = 0.0;
+#pragma unroll 2
+  for (int l = 0; l < F; l++) {
+    const double2 t = tab[idx];
+    idx += step;
+    if (idx >= M) idx -= M;
+#pragma unroll
+    for (int r = 0; r < ZOOM_R; r++) {
+      const double2 f = row[r][l];
+      sr[r] += f.x * t.x - f.y * t.y;
+      si[r] += f.x * t.y + f.y * t.x;
+    }
   }
-  const int y = kyi / Q, yf = kyi - y * Q;
-  const int x = kxi / Q, xf = kxi - x * Q;
-  const int64_t o = out_off[p] + (((int64_t)yf * Q + xf) * S + y) * S + x;
-  out[o].x = sr;
-  out[o].y = si;
+  if (i >= QS) return;
+#pragma unroll
+  for (int r = 0; r < ZOOM_R; r++)
+    if (m0 + r < F)
+      tmp[p * tmp_stride + (int64_t)(m0 + r) * QS + i] = make_double2(sr[r], si[r]);
+}
+
+// Column pass into [yf][xf][y][x]: rows ky = Q y + yf.
+template <typename OutT>
+__global__ __launch_bounds__(ZOOM_NT) void k_zoom_cols(
+    const double2 *__restrict__ tmp, int64_t tmp_stride, int F, int Q,
+    const int32_t *__restrict__ Sp, const int64_t *__restrict__ out_off,
+    const double2 *__restrict__ tab, OutT *__restrict__ out) {
+  const int p = blockIdx.z;
+  const int S = Sp[p], QS = Q * S;
+  const uint32_t M = (uint32_t)F * (uint32_t)Q;  // below 2^31
+  const int k0 = zoom_wave_rows(blockIdx.y);
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (blockIdx.x * 64 >= QS || k0 >= QS) return;
+  const double2 *col = tmp + p * tmp_stride + min(i, QS - 1);
+  uint32_t idx[ZOOM_R], step[ZOOM_R];
+  double sr[ZOOM_R], si[ZOOM_R];
+#pragma unroll
+  for (int r = 0; r < ZOOM_R; r++) {
+    const int64_t k = (int64_t)min(k0 + r, QS - 1) - (int64_t)Q * (S / 2);
+    idx[r] = (uint32_t)mod64(-k * (F / 2), M);
+    step[r] = (uint32_t)mod64(k, M);
+    sr[r] = si[r] = 0.0;
+  }
+#pragma unroll 2
+  for (int m = 0; m < F; m++) {
+    const double2 f = col[(int64_t)m * QS];
+#pragma unroll
+    for (int r = 0; r < ZOOM_R; r++) {
+      const double2 t = tab[idx[r]];
+      sr[r] += f.x * t.x - f.y * t.y;
+      si[r] += f.x * t.y + f.y * t.x;
+      idx[r] += step[r];
+      if (idx[r] >= M) idx[r] -= M;
+    }
+  }
+  if (i >= QS) return;
+  const int xf = i / S, x = i - xf * S;
+#pragma unroll
+  for (int r = 0; r < ZOOM_R; r++) {
+    const int ky = k0 + r;
+    if (ky >= QS) break;
+    const int y = ky / Q, yf = ky - y * Q;
+    const int64_t o = out_off[p] + (((int64_t)yf * Q + xf) * S + y) * S + x;
+    out[o].x = sr[r];
+    out[o].y = si[r];
+  }
 }
 
 // 1D: out[xf][x] = sum_l ff[l] E(Q x + xf - Q(S//2), l); one workgroup per
@@ -185,19 +243,27 @@ int oversample_planes(croc_ctx *ctx, const double2 *ff, int64_t ff_stride,
                       const int64_t *dOff, void *out, int out_double) {
   const int64_t maxQS = (int64_t)Q * maxS;
   const int64_t tmp_stride = (int64_t)F * maxQS;
-  double2 *tmp = (double2 *)ws_get(ctx, WS_TMP,
-                                   sizeof(double2) * tmp_stride * nplanes);
-  if (!tmp) return CROC_ENOMEM;
+  const int64_t M = (int64_t)F * Q;
+  CROC_REQUIRE(M <= INT32_MAX, CROC_EINVAL, "oversampled far field of %lld samples",
+               (long long)M);
+  // the twiddle table, then the intermediate
+  double2 *tab =
+      (double2 *)ws_get(ctx, WS_TMP, sizeof(double2) * ((size_t)M + tmp_stride * nplanes));
+  if (!tab) return CROC_ENOMEM;
+  double2 *tmp = tab + M;
   hipStream_t s = ctx->stream;
-  dim3 g1((unsigned)((tmp_stride + 255) / 256), nplanes);
-  k_zoom_rows<<<g1, 256, 0, s>>>(ff, ff_stride, F, Q, dS, tmp, tmp_stride);
-  dim3 g2((unsigned)((maxQS * maxQS + 255) / 256), nplanes);
+  k_twiddles<<<(unsigned)((M + 255) / 256), 256, 0, s>>>(M, tab);
+  const int64_t rows = ZOOM_R * (ZOOM_NT / 64);
+  const unsigned nx = (unsigned)((maxQS + 63) / 64);
+  k_zoom_rows<<<dim3(nx, (unsigned)((F + rows - 1) / rows), nplanes), ZOOM_NT, 0, s>>>(
+      ff, ff_stride, F, Q, dS, tab, tmp, tmp_stride);
+  const dim3 g2(nx, (unsigned)((maxQS + rows - 1) / rows), nplanes);
   if (out_double)
-    k_zoom_cols<double2><<<g2, 256, 0, s>>>(tmp, tmp_stride, F, Q, dS, dOff,
-                                            (double2 *)out);
+    k_zoom_cols<double2><<<g2, ZOOM_NT, 0, s>>>(tmp, tmp_stride, F, Q, dS, dOff, tab,
+                                                (double2 *)out);
   else
-    k_zoom_cols<float2><<<g2, 256, 0, s>>>(tmp, tmp_stride, F, Q, dS, dOff,
-                                           (float2 *)out);
+    k_zoom_cols<float2><<<g2, ZOOM_NT, 0, s>>>(tmp, tmp_stride, F, Q, dS, dOff, tab,
+                                               (float2 *)out);
   CROC_HIP(hipGetLastError());
   return CROC_OK;
 }

@@ -152,3 +152,21 @@ def test_aw_fft_speed(gpu, S):
         out[name] = (time.perf_counter() - t0) / 8 * 1e3
     print('AW kernel set S=%d (1024 sub-kernels): fft %.3f ms, direct %.3f ms'
           % (S, out['fft'], out['uncached']), flush=True)
+
+
+@pytest.mark.parametrize('F,Q,supports', [(9, 1, [9]), (17, 3, [1, 2, 16]), (32, 8, [31, 8]),
+                                          (33, 5, [13, 32]), (64, 16, [4, 5])])
+def test_w_kernel_bank_edges(gpu, F, Q, supports):
+    """Far fields and kernels off the sizes of the kernel generator's row
+    groups (8 and 32 rows) and column blocks (64), planes of different
+    supports in one launch.  Bound: F^2 unit terms summed in two passes of F,
+    each term a few roundings: (2 F + 16) eps F^2."""
+    ws = [3.5 * (k - 1) for k in range(len(supports))]
+    for invert in (True, False):
+        bank = G.w_kernel_bank(0.3, ws, F, supports, Q, invert, double=True)
+        got = bank.kern.cpu().numpy()
+        for k, S in enumerate(supports):
+            ref = R.w_kernel(0.3, ws[k], F, S, Q, invert=invert)
+            o = int(bank.plane_off_h[k])
+            err = numpy.abs(got[o:o + ref.size].reshape(ref.shape) - ref).max()
+            assert err <= (2 * F + 16) * 2.3e-16 * F * F, (F, Q, S, err)
