@@ -12,6 +12,8 @@
 // coordinate p whose synthesis.py frac_coord gives the same cell and
 // sub-offset, so the tile path lands each visibility exactly where grid.c
 // does.
+#include <algorithm>
+
 #include "internal.h"
 
 namespace {
@@ -33,11 +35,25 @@ BlView view(const croc_bl_set *s) {
                 s->vis_first,  s->uvw_m,      s->freq,       (float2 *)s->vis};
 }
 
+// x / c rounded as IEEE division rounds it, in four operations: the product
+// with the rounded reciprocal (off by 2^-55.4 relative, so the product lies
+// within 0.69 ulp of the quotient), corrected by the exact remainder, which
+// then rounds correctly (Markstein, IBM J. Res. Dev. 34 (1990): q faithful,
+// reciprocal correctly rounded).  Values whose remainder could underflow or
+// overflow divide.
+__device__ __forceinline__ double over_c(double x) {
+  constexpr double RC = 1.0 / C_LIGHT;
+  const double ax = fabs(x);
+  if (!(ax >= 1e-250 && ax <= 1e250)) return x / C_LIGHT;
+  const double q = x * RC;
+  return fma(fma(-q, C_LIGHT, x), RC, q);
+}
+
 // grid.h:53-60: uvw_m * f / c, the product rounded before the division.
 __device__ __forceinline__ double bl_lambda(const BlView &s, int64_t row, int64_t fi, int k) {
 #pragma clang fp contract(off)
   const double prod = s.uvw_m[3 * row + k] * s.freq[fi];
-  return prod / C_LIGHT;
+  return over_c(prod);
 }
 
 // grid.c:35-53 for x = theta * u: ox = rint((N/2 - x) Q), cell N - ox/Q,
@@ -45,24 +61,26 @@ __device__ __forceinline__ double bl_lambda(const BlView &s, int64_t row, int64_
 // grid's upper edge (ox < 0: a negative sub-offset) or so far outside that
 // no grid of at most 65536 cells with Q <= 2^20 could hold it.  The
 // quotient comes from the FP64 reciprocal of Q (within 2^-12 of the true
-// quotient for ox < 2^40), corrected by the remainder: exact.
-__device__ __forceinline__ bool frac_coord_c(int N, int Q, double x, int64_t *ix, int *fx) {
+// quotient for ox < 2^40), corrected by the remainder: exact, all in FP64
+// integers below 2^53.
+__device__ __forceinline__ bool frac_coord_c(int N, int Q, double x, int *ix, int *fx) {
 #pragma clang fp contract(off)
-  const double s = ((double)(N / 2) - x) * (double)Q;
+  const double dq = (double)Q;
+  const double s = ((double)(N / 2) - x) * dq;
   if (!(fabs(s) < 0x1p40)) return false;
   const double so = rint(s);
   if (so < 0.0) return false;
-  const int64_t ox = (int64_t)so;
-  int64_t q = (int64_t)(so * (1.0 / (double)Q));
-  int64_t rem = ox - q * Q;
-  if (rem < 0) {
-    q -= 1;
-    rem += Q;
-  } else if (rem >= Q) {
-    q += 1;
-    rem -= Q;
+  double q = trunc(so * (1.0 / dq));
+  double rem = fma(-q, dq, so);
+  if (rem < 0.0) {
+    q -= 1.0;
+    rem += dq;
+  } else if (rem >= dq) {
+    q += 1.0;
+    rem -= dq;
   }
-  *ix = (int64_t)N - q;
+  if (q > 0x1p30) return false;  // the cell N - q lies far below the grid
+  *ix = N - (int)q;
   *fx = (int)rem;
   return true;
 }
@@ -72,13 +90,13 @@ __device__ __forceinline__ bool frac_coord_c(int N, int Q, double x, int64_t *ix
 __device__ __forceinline__ bool bl_window(int N, int Q, int S, double theta, double u, double v,
                                           int *x0, int *y0, int *fx, int *fy) {
 #pragma clang fp contract(off)
-  int64_t ix, iy;
+  int ix, iy;
   if (!frac_coord_c(N, Q, theta * u, &ix, fx) || !frac_coord_c(N, Q, theta * v, &iy, fy))
     return false;
-  const int64_t ax = ix - S / 2, ay = iy - S / 2;
+  const int ax = ix - S / 2, ay = iy - S / 2;
   if (ax < 0 || ay < 0 || ax + S > N || ay + S > N) return false;
-  *x0 = (int)ax;
-  *y0 = (int)ay;
+  *x0 = ax;
+  *y0 = ay;
   return true;
 }
 
@@ -247,10 +265,10 @@ struct DegridArgs {
   int N, S, Q;
   double theta;
   const double *kern;  // real [Q][S]
-  const float *kf;     // the same rounded to FP32 (degrid pass)
+  const float *kf;     // the same rounded to FP32, rows padded with zeros (degrid pass)
   float2 *out;
   unsigned long long *count;  // [n chunks] degridded visibilities
-  unsigned long long *total;  // their sum
+  unsigned long long *total;  // their sum (check pass)
   int count_in_degrid;        // counts made by the degrid pass (else the check pass)
   uint32_t *status;
 };
@@ -274,6 +292,19 @@ __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long x
   return t;
 }
 
+// j / n and j % n of a visibility index of a chunk (n > 0): 32-bit division
+// when the chunk allows it, a fraction of the 64-bit one's instructions.
+__device__ __forceinline__ void split_index(int64_t j, int n, bool small, int *t, int *f) {
+  if (small) {
+    const uint32_t q = (uint32_t)j / (uint32_t)n;
+    *t = (int)q;
+    *f = (int)((uint32_t)j - q * (uint32_t)n);
+  } else {
+    *t = (int)(j / n);
+    *f = (int)(j % n);
+  }
+}
+
 // Validation pass: ranges, windows, per-chunk counts.  Nothing written but
 // counts and status.
 __global__ __launch_bounds__(BL_NT) void k_bl_degrid_check(DegridArgs a) {
@@ -290,9 +321,10 @@ __global__ __launch_bounds__(BL_NT) void k_bl_degrid_check(DegridArgs a) {
       const int nfw = r.f1 - r.f0;
       const int64_t m = (int64_t)(r.t1 - r.t0) * nfw;
       for (int64_t j = threadIdx.x; j < m; j += BL_NT) {
-        const int t = r.t0 + (int)(j / nfw), f = r.f0 + (int)(j % nfw);
+        int t, f;
+        split_index(j, nfw, m <= INT32_MAX, &t, &f);
         double u, v, pu, pv;
-        chunk_uv(a.s, a.c, r, t, f, &u, &v);
+        chunk_uv(a.s, a.c, r, r.t0 + t, r.f0 + f, &u, &v);
         const int kind = classify(box, u, v, &pu, &pv);
         if (kind == 1 || kind == 2) {
           int x0, y0, fx, fy;
@@ -317,102 +349,294 @@ __global__ void k_bl_chunk_check(DegridArgs a) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.c.n) return;
   const Chunk r = chunk_at(a.s, a.c, k);
-  a.count[k] = 0;
   if (!r.ok) atomicOr(a.status, (uint32_t)ST_RANGE);
 }
 
-// Degridding.  Each wavefront takes 64 consecutive visibilities of a chunk:
-// first every lane works out the coordinates of one of them (FP64 uvw
-// scaling, window rule, frac_coord), then groups of G lanes (G a power of
-// two >= S) degrid them, 64 / G at a time, fetching each visibility's
-// window, sub-offsets and output index from the lane that computed them.
-// In a group, lane x sums column x of the window over the rows weighted by
-// k[fy][y]; the group then sums the columns weighted by k[fx][x].  Rows are
-// read as S consecutive complex64 cells.  FP32 arithmetic on the table's
-// values rounded to FP32 (kf).
-template <int G>
+// Minimum / maximum over the wavefront (values of lanes outside are the
+// identity): DPP butterflies within rows of 16, then the row broadcasts.
+template <bool MAX>
+__device__ __forceinline__ int wave_extreme(int v) {
+  constexpr int ID = MAX ? INT32_MIN : INT32_MAX;
+  auto op = [](int p, int q) { return MAX ? max(p, q) : min(p, q); };
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0xb1, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0x4e, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0x141, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0x140, 0xf, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0x142, 0xa, 0xf, false));
+  v = op(v, __builtin_amdgcn_update_dpp(ID, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Degridding, one workgroup per chunk.  Each wavefront takes 64 consecutive
+// visibilities of the chunk: first every lane works out the coordinates of
+// one of them (FP64 uvw scaling, window rule, frac_coord).  Their windows
+// mostly overlap -- neighbouring channels of a dump move by a fraction of a
+// cell -- so the wavefront stages the windows' bounding box in LDS (at most
+// BL_BOX cells; all 64 visibilities, else the channels of one dump at a time)
+// and every lane sums its own window from there.  Supports above 16 and
+// boxes that do not fit take the grid directly: groups of L = G / W lanes (G a
+// power of two >= S) degrid the visibilities, 64 / L at a time, fetching
+// each one's window and sub-offsets from the lane that computed them and
+// handing the sum back to it; in a group, lane x sums columns W x .. W x + W
+// - 1.  Either way a column is summed over the rows weighted by k[fy][y],
+// the pairs of columns weighted by k[fx][x] are summed and the pairs' sums added
+// as a butterfly, so both give the same value bit for bit.  The stores are
+// one coalesced write per 64 visibilities.  FP32 arithmetic on the table's
+// values rounded to FP32 (kf, row pitch G).
+//
+// stream32k with 128 stations (66.6e6 visibilities, S = 8): one column per lane
+// from memory took 4.38 ms, pairs of columns (16-byte loads) 2.26 ms, bound by
+// L1 accesses (90 % of the cycles, ~18 per visibility, each row straddling
+// two 64-byte lines); from the LDS box 2.1
+// ms.
+constexpr int BL_BOX = 600;  // cells per wavefront: 19 KiB a workgroup
+typedef float bl_cell2 __attribute__((ext_vector_type(4), aligned(8)));  // two cells
+
+template <int G, int W>
 __global__ __launch_bounds__(BL_NT) void k_bl_degrid(DegridArgs a) {
-  constexpr int V = 64 / G;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int x = lane & (G - 1), grp = lane / G;
+  constexpr int L = G / W, V = 64 / L;
+  constexpr int RB = G < 16 ? G : 16;  // rows whose loads are in flight together
+  constexpr bool BOX = G <= 16 && W == 2;
+  __shared__ unsigned int s_n[BL_NT / 64];
+  __shared__ float2 s_box[BOX ? BL_NT / 64 : 1][BOX ? BL_BOX + G : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int x = lane & (L - 1), grp = lane / L;
   const int S = a.S, N = a.N;
-  unsigned long long tot = 0;
+  // the lane's first column: odd supports end on the pair (S - 2, S - 1)
+  const int col = W * x;
+  const int c0 = W == 1 ? min(col, S - 1) : min(col, S - 2);
+  const bool has = col < S, odd = W == 2 && col == S - 1;
   for (int64_t k = blockIdx.x; k < a.c.n; k += gridDim.x) {
     const Chunk r = chunk_at(a.s, a.c, k);
     const Box box = chunk_box(a, r);
     const float2 *grid = a.grid + (int64_t)r.sub * N * N;
     const int nfw = r.f1 - r.f0;
     const int64_t m = (int64_t)(r.t1 - r.t0) * nfw;
-    unsigned long long nk = 0;
+    const bool small = m <= INT32_MAX;
+    unsigned int nk = 0;
     for (int64_t jb = (int64_t)wave * 64; jb < m; jb += BL_NT) {
       // this lane's visibility: window origin, sub-offsets, kind, output
       uint32_t xy = 0u, fxv = 0u, kfy = 0u;
       int64_t o = 0;
+      int kind = 0, t = 0;
       const int64_t j = jb + lane;
       if (j < m) {
-        const int t = r.t0 + (int)(j / nfw), f = r.f0 + (int)(j % nfw);
-        o = r.out0 + (int64_t)(t - r.t0) * r.orow + (f - r.f0);
+        int f;
+        split_index(j, nfw, small, &t, &f);
+        o = r.out0 + (int64_t)t * r.orow + f;
         double u, v, pu, pv;
-        chunk_uv(a.s, a.c, r, t, f, &u, &v);
-        const int kind = classify(box, u, v, &pu, &pv);
+        chunk_uv(a.s, a.c, r, r.t0 + t, r.f0 + f, &u, &v);
+        kind = classify(box, u, v, &pu, &pv);
         int x0 = 0, y0 = 0, fx = 0, fy = 0;
-        if (kind == 1 || kind == 2) bl_window(N, a.Q, S, a.theta, pu, pv, &x0, &y0, &fx, &fy);
+        const bool deg = kind == 1 || kind == 2;
+        if (deg) bl_window(N, a.Q, S, a.theta, pu, pv, &x0, &y0, &fx, &fy);
         xy = (uint32_t)x0 | ((uint32_t)y0 << 16);
         fxv = (uint32_t)fx;
-        kfy = (uint32_t)fy | ((uint32_t)kind << 28);
+        kfy = (uint32_t)fy | (deg ? 0x80000000u : 0u);
       }
-      nk += (unsigned long long)__popcll(__ballot((kfy >> 28) == 1u || (kfy >> 28) == 2u));
-      const int nr = (int)((min<int64_t>(64, m - jb) + V - 1) / V);  // wave-uniform
-      for (int rr = 0; rr < nr; rr++) {
+      const unsigned long long degs = __ballot((kfy >> 31) != 0u);
+      nk += (unsigned int)__popcll(degs);
+      float2 res = make_float2(0.f, 0.f);
+      unsigned long long left = degs;
+      if constexpr (BOX) {
+        float2 *box_w = s_box[wave];
+        const int x0 = (int)(xy & 0xffffu), y0 = (int)(xy >> 16);
+        const float4 *ky4 = (const float4 *)(a.kf + (int64_t)G * (kfy & 0x7fffffffu));
+        const float4 *kx4 = (const float4 *)(a.kf + (int64_t)G * fxv);
+        float4 ky[G / 4], kx[G / 4];
+#pragma unroll
+        for (int i = 0; i < G / 4; i++) {
+          ky[i] = ky4[i];
+          kx[i] = kx4[i];
+        }
+        while (left) {
+          unsigned long long mask = left;
+          int xmin, ymin, bw, bh, pitch;
+          auto bounds = [&]() {
+            const bool mine = (mask >> lane) & 1ull;
+            xmin = wave_extreme<false>(mine ? x0 : INT32_MAX);
+            ymin = wave_extreme<false>(mine ? y0 : INT32_MAX);
+            bw = wave_extreme<true>(mine ? x0 : INT32_MIN) - xmin + S;
+            bh = wave_extreme<true>(mine ? y0 : INT32_MIN) - ymin + S;
+            pitch = bw | 1;  // rows on different banks
+            return bh * pitch <= BL_BOX;
+          };
+          if (!bounds()) {  // one dump of the batch, if it holds enough of it
+            const int lead = __builtin_amdgcn_readlane(t, __ffsll((long long)left) - 1);
+            mask = left & __ballot(t == lead);
+            if (__popcll(mask) < 16 || !bounds()) break;
+          }
+          left &= ~mask;
+          // the box, eight loads of 64 cells in flight (cell i at row i / bw,
+          // exact in FP32 for i < 2^12)
+          const int n = bh * bw;
+          const float2 *corner = grid + (int64_t)ymin * N + xmin;
+          const float inv = 1.0f / (float)bw;
+          for (int i0 = 0; i0 < n; i0 += 512) {
+            float2 g[8];
+            int at[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+              if (i0 + 64 * u < n) {  // wave-uniform
+                const int i = min(i0 + 64 * u + lane, n - 1);
+                const int yy = (int)(((float)i + 0.5f) * inv), xx = i - yy * bw;
+                g[u] = corner[(int64_t)yy * N + xx];
+                at[u] = yy * pitch + xx;
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+              if (i0 + 64 * u < n) box_w[at[u]] = g[u];
+          }
+          // this wavefront alone reads its box, and its LDS operations are
+          // carried out in order: only the compiler has to keep that order
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          if ((mask >> lane) & 1ull) {
+            const float2 *cell = box_w + (y0 - ymin) * pitch + (x0 - xmin);
+            float sr[G], si[G];
+#pragma unroll
+            for (int c = 0; c < G; c++) sr[c] = si[c] = 0.f;
+            // rows past S re-read row S - 1 with weight 0; columns past S read
+            // on in the box (or its padding) into sums that are not used
+#pragma unroll
+            for (int y = 0; y < G; y++) {
+              const float2 *row = cell + min(y, S - 1) * pitch;
+              float2 g[G];
+#pragma unroll
+              for (int c = 0; c < G; c++) g[c] = row[c];
+              const float wy = y % 4 == 0 ? ky[y / 4].x : y % 4 == 1 ? ky[y / 4].y
+                             : y % 4 == 2 ? ky[y / 4].z : ky[y / 4].w;
+#pragma unroll
+              for (int c = 0; c < G; c++) {
+                sr[c] = fmaf(wy, g[c].x, sr[c]);
+                si[c] = fmaf(wy, g[c].y, si[c]);
+              }
+            }
+            // pairs of columns, then the butterfly of the group path
+            float pr[L], pi[L];
+#pragma unroll
+            for (int i = 0; i < L; i++) {
+              const float wa = i % 2 ? kx[i / 2].z : kx[i / 2].x;
+              const float wb = i % 2 ? kx[i / 2].w : kx[i / 2].y;
+              const bool one = 2 * i == S - 1, none = 2 * i >= S;
+              pr[i] = none ? 0.f : one ? wa * sr[2 * i] : fmaf(wb, sr[2 * i + 1], wa * sr[2 * i]);
+              pi[i] = none ? 0.f : one ? wa * si[2 * i] : fmaf(wb, si[2 * i + 1], wa * si[2 * i]);
+            }
+#pragma unroll
+            for (int w = L / 2; w > 0; w >>= 1) {
+#pragma unroll
+              for (int i = 0; i < w; i++) {
+                pr[i] += pr[i + w];
+                pi[i] += pi[i + w];
+              }
+            }
+            res = make_float2(pr[0], pi[0]);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();  // the box is read before it is rewritten
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+      }
+#pragma unroll 1
+      for (int rr = 0; rr < 64 / V; rr++) {
+        // rounds without a visibility left are skipped
+        if (((left >> (rr * V)) & ((1ull << V) - 1ull)) == 0ull) continue;
         const int q = rr * V + grp;
         const uint32_t xy_q = __shfl(xy, q), fx_q = __shfl(fxv, q), kfy_q = __shfl(kfy, q);
-        const uint32_t olo = __shfl((uint32_t)o, q), ohi = __shfl((uint32_t)(o >> 32), q);
-        const int kind = (int)(kfy_q >> 28);
         float ar = 0.f, ai = 0.f;
-        if ((kind == 1 || kind == 2) && x < S) {
+        if (((left >> q) & 1ull) && has) {
           const int x0 = (int)(xy_q & 0xffffu), y0 = (int)(xy_q >> 16);
-          const float2 *col = grid + (int64_t)y0 * N + x0 + x;
-          const float *ky = a.kf + (int64_t)S * (kfy_q & 0xfffffffu);
-          // all G row loads issue before the products: rows past S re-read
-          // row S - 1 (in the window) with weight 0
-          float2 g[G];
-          float w[G];
+          const float2 *cell = grid + (int64_t)y0 * N + x0 + c0;
+          const float4 *ky = (const float4 *)(a.kf + (int64_t)G * (kfy_q & 0x7fffffffu));
+          const float *kx = a.kf + (int64_t)G * fx_q + col;
+          // rows past S re-read row S - 1 (in the window) with weight 0
+          float s[2 * W];
 #pragma unroll
-          for (int y = 0; y < G; y++) {
-            const int yy = y < S ? y : S - 1;
-            g[y] = col[(int64_t)yy * N];
-            w[y] = y < S ? ky[yy] : 0.f;
-          }
+          for (int i = 0; i < 2 * W; i++) s[i] = 0.f;
 #pragma unroll
-          for (int y = 0; y < G; y++) {
-            ar = fmaf(w[y], g[y].x, ar);
-            ai = fmaf(w[y], g[y].y, ai);
+          for (int yb = 0; yb < G; yb += RB) {
+            float4 w[RB / 4];
+#pragma unroll
+            for (int i = 0; i < RB / 4; i++) w[i] = ky[yb / 4 + i];
+            float g[RB][2 * W];
+#pragma unroll
+            for (int y = 0; y < RB; y++) {
+              const float2 *p = cell + (int64_t)min(yb + y, S - 1) * N;
+              if constexpr (W == 2) {
+                const bl_cell2 c = *(const bl_cell2 *)p;
+                g[y][0] = c.x;
+                g[y][1] = c.y;
+                g[y][2] = c.z;
+                g[y][3] = c.w;
+              } else {
+                const float2 c = *p;
+                g[y][0] = c.x;
+                g[y][1] = c.y;
+              }
+            }
+#pragma unroll
+            for (int y = 0; y < RB; y++) {
+              const float4 w4 = w[y / 4];
+              const float wy = y % 4 == 0 ? w4.x : y % 4 == 1 ? w4.y : y % 4 == 2 ? w4.z : w4.w;
+#pragma unroll
+              for (int i = 0; i < 2 * W; i++) s[i] = fmaf(wy, g[y][i], s[i]);
+            }
           }
-          const float kx = a.kf[(int64_t)S * fx_q + x];
-          ar *= kx;
-          ai *= kx;
+          if constexpr (W == 2) {
+            const float2 wx = *(const float2 *)kx;
+            ar = odd ? wx.x * s[2] : fmaf(wx.y, s[2], wx.x * s[0]);
+            ai = odd ? wx.x * s[3] : fmaf(wx.y, s[3], wx.x * s[1]);
+          } else {
+            ar = kx[0] * s[0];
+            ai = kx[0] * s[1];
+          }
         }
 #pragma unroll
-        for (int w = G / 2; w > 0; w >>= 1) {
+        for (int w = L / 2; w > 0; w >>= 1) {
           ar += __shfl_xor(ar, w);
           ai += __shfl_xor(ai, w);
         }
-        if (x == 0 && kind != 0) {
-          const int64_t oq = (int64_t)(((uint64_t)ohi << 32) | olo);
-          a.out[oq] = kind == 3 ? make_float2(0.f, 0.f)
-                                : make_float2(ar, kind == 2 ? -ai : ai);
-        }
+        // every lane of a group holds its sum; lane rr V + g owns group g's
+        const float br = __shfl(ar, (lane & (V - 1)) * L), bi = __shfl(ai, (lane & (V - 1)) * L);
+        if (lane / V == rr && ((left >> lane) & 1ull)) res = make_float2(br, bi);
       }
+      if (kind != 0)
+        a.out[o] = kind == 3 ? make_float2(0.f, 0.f)
+                             : make_float2(res.x, kind == 2 ? -res.y : res.y);
     }
-    if (a.count_in_degrid && lane == 0 && nk) atomicAdd(&a.count[k], nk);
-    tot += nk;
+    if (a.count_in_degrid) {
+      if (lane == 0) s_n[wave] = nk;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        unsigned long long n = 0;
+        for (int w = 0; w < BL_NT / 64; w++) n += s_n[w];
+        a.count[k] = n;
+      }
+      __syncthreads();
+    }
   }
-  if (a.count_in_degrid && lane == 0 && tot) atomicAdd(a.total, tot);
 }
 
-__global__ void k_to_float(const double *in, float *out, int64_t n) {
+// *total = sum of count[0 .. n - 1].
+__global__ __launch_bounds__(1024) void k_bl_total(const unsigned long long *__restrict__ count,
+                                                   int64_t n, unsigned long long *total) {
+  __shared__ unsigned long long red[1024 / 64];
+  unsigned long long s = 0;
+  for (int64_t i = threadIdx.x; i < n; i += 1024) s += count[i];
+  s = block_sum_u64(s, red);
+  if (threadIdx.x == 0) *total = s;
+}
+
+// out[row][0 .. pitch - 1] = in[row][0 .. S - 1] rounded, zeros past S.
+__global__ void k_to_float(const double *in, float *out, int64_t rows, int S, int pitch) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (float)in[i];
+  if (i >= rows * pitch) return;
+  const int64_t r = i / pitch;
+  const int c = (int)(i - r * pitch);
+  out[i] = c < S ? (float)in[r * S + c] : 0.f;
 }
 
 // ---------------------------------------------------------------------------
@@ -652,38 +876,45 @@ int degrid_run(croc_ctx *ctx, DegridArgs a, bool safe, uint64_t *ndeg_total) {
     if (!a.count) return CROC_ENOMEM;
   }
   a.count_in_degrid = safe ? 1 : 0;
-  const int nb = blocks_for(ctx, a.c.n);
+  const int nb = (int)std::min<int64_t>(a.c.n, 1 << 20);  // a workgroup per chunk
   if (safe)
     k_bl_chunk_check<<<(unsigned)((a.c.n + 255) / 256), 256, 0, ctx->stream>>>(a);
   else
-    k_bl_degrid_check<<<nb, BL_NT, 0, ctx->stream>>>(a);
+    k_bl_degrid_check<<<blocks_for(ctx, a.c.n), BL_NT, 0, ctx->stream>>>(a);
   if ((rc = read_word(ctx, st))) return rc;
+  const int S = a.S;
+  const int G = S <= 4 ? 4 : S <= 8 ? 8 : S <= 16 ? 16 : S <= 32 ? 32 : 64;
   {
-    const int64_t nk = (int64_t)a.Q * a.S;
+    const int64_t nk = (int64_t)a.Q * G;
     float *kf = (float *)ws_get(ctx, WS_BL_BANK, sizeof(float) * nk);
     if (!kf) return CROC_ENOMEM;
-    k_to_float<<<(unsigned)((nk + 255) / 256), 256, 0, ctx->stream>>>(a.kern, kf, nk);
+    k_to_float<<<(unsigned)((nk + 255) / 256), 256, 0, ctx->stream>>>(a.kern, kf, a.Q, S, G);
     a.kf = kf;
   }
   CROC_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
   tap_timer_reset(ctx, 1);
   if ((rc = tap_timer_begin(ctx, 1))) return rc;
-  const int S = a.S;
-  if (S <= 4)
-    k_bl_degrid<4><<<nb, BL_NT, 0, ctx->stream>>>(a);
-  else if (S <= 8)
-    k_bl_degrid<8><<<nb, BL_NT, 0, ctx->stream>>>(a);
-  else if (S <= 16)
-    k_bl_degrid<16><<<nb, BL_NT, 0, ctx->stream>>>(a);
-  else if (S <= 32)
-    k_bl_degrid<32><<<nb, BL_NT, 0, ctx->stream>>>(a);
+  if (S == 1)  // no pair of columns to read
+    k_bl_degrid<4, 1><<<nb, BL_NT, 0, ctx->stream>>>(a);
+  else if (G == 4)
+    k_bl_degrid<4, 2><<<nb, BL_NT, 0, ctx->stream>>>(a);
+  else if (G == 8)
+    k_bl_degrid<8, 2><<<nb, BL_NT, 0, ctx->stream>>>(a);
+  else if (G == 16)
+    k_bl_degrid<16, 2><<<nb, BL_NT, 0, ctx->stream>>>(a);
+  else if (G == 32)
+    k_bl_degrid<32, 2><<<nb, BL_NT, 0, ctx->stream>>>(a);
   else
-    k_bl_degrid<64><<<nb, BL_NT, 0, ctx->stream>>>(a);
+    k_bl_degrid<64, 2><<<nb, BL_NT, 0, ctx->stream>>>(a);
   CROC_HIP(hipGetLastError());
   if ((rc = tap_timer_end(ctx, 1))) return rc;
   CROC_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
   ctx->ev_degrid = true;
   if (ndeg_total) {
+    if (safe) {
+      k_bl_total<<<1, 1024, 0, ctx->stream>>>(a.count, a.c.n, a.total);
+      CROC_HIP(hipGetLastError());
+    }
     unsigned long long t = 0;
     CROC_HIP(hipMemcpyAsync(&t, a.total, sizeof(t), hipMemcpyDeviceToHost, ctx->stream));
     CROC_HIP(hipStreamSynchronize(ctx->stream));

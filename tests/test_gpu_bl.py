@@ -355,3 +355,31 @@ def test_streamer_windows_near_subgrid_edge(gpu):
         BL.streamer_degrid_worker(dev, subd, xM, theta, 0.0, 0.0, chunks, *box,
                                   BL.SepKernelData(kern), tc, fc, vis_queue=queue)
     assert bool((queue == 5.0).all())
+
+
+@pytest.mark.parametrize('S', [1, 2, 3, 5, 8, 11, 16, 17])
+def test_degrid_boxes_and_groups_agree(gpu, S):
+    """Clustered visibilities (their windows staged as one box) and the same
+    ones scattered among others (lane groups on the grid) degrid to the same
+    bits, with windows on the grid's first and last cells; both within
+    (S^2 + 8) FP32 roundings of the sum of absolute products."""
+    rng = numpy.random.default_rng(100 + S)
+    N, theta, Q, n = 96, 0.02, 16, 192
+    g, gd = rand_grid(rng, N)
+    kern = rng.normal(size=(Q, S))
+    lo, hi = -N // 2 + S // 2, N - N // 2 - (S - S // 2)   # cells of the extreme windows
+    cl = [(lo + rng.uniform(0, 3, n), lo + rng.uniform(0, 3, n)),
+          (hi - rng.uniform(0, 3, n), hi - rng.uniform(0, 3, n)),
+          (rng.uniform(-2, 2, n), hi - rng.uniform(0, 3, n))]
+    u = numpy.concatenate([c[0] for c in cl]) / theta
+    v = numpy.concatenate([c[1] for c in cl]) / theta
+    k = BL.SepKernelData(kern)
+    ordered = BL.degrid_conv_uv(gd, N, theta, u, v, k).cpu().numpy()
+    mix = rng.permutation(len(u))
+    mixed = BL.degrid_conv_uv(gd, N, theta, u[mix], v[mix], k).cpu().numpy()
+    assert_array_equal(ordered[mix], mixed)
+    uv = numpy.stack([u, v], 1)
+    ref = B.degrid_conv_uv(g, theta, uv, kern)
+    size = B.degrid_conv_uv(numpy.abs(g.real) + numpy.abs(g.imag) + 0j, theta, uv,
+                            numpy.abs(kern)).real
+    assert (numpy.abs(ordered - ref) <= (S * S + 8) * 2.0 ** -24 * size).all()
