@@ -43,37 +43,75 @@ __device__ __forceinline__ float2 rotate(float2 v, double kf, double phi) {
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 
-// cos / sin of 2 pi k / 16, k = 0..7 (rounded from FP64).
-__device__ constexpr float C16[8] = {1.0f, 0.92387953251128674f, 0.70710678118654757f,
-                                      0.38268343236508984f, 0.0f, -0.38268343236508973f,
-                                      -0.70710678118654746f, -0.92387953251128674f};
-__device__ constexpr float S16[8] = {0.0f, 0.38268343236508978f, 0.70710678118654746f,
-                                      0.92387953251128674f, 1.0f, 0.92387953251128674f,
-                                      0.70710678118654757f, 0.38268343236508989f};
+// v sqrt(1/2) (1 + s i) and v sqrt(1/2) (-1 + s i): the odd eighths of a turn.
+__device__ __forceinline__ float2 rot45(float2 v, float s) {
+  constexpr float H = 0.70710678118654757f;
+  return make_float2(H * fmaf(-s, v.y, v.x), H * fmaf(s, v.x, v.y));
+}
+__device__ __forceinline__ float2 rot135(float2 v, float s) {
+  constexpr float H = 0.70710678118654757f;
+  return make_float2(-H * fmaf(s, v.y, v.x), H * fmaf(s, v.x, -v.y));
+}
 
-// In-register radix-2 DFT of N <= 16 points: v[k] = sum_j v[j] W_N^(jk),
-// W_N = exp(sgn 2 pi i / N).
+// Four-point DFT in place, W_4 = s i (s = sgn).
+__device__ __forceinline__ void fft_reg4(float2 &a, float2 &b, float2 &c, float2 &d, float s) {
+  const float2 p = cadd(a, c), q = csub(a, c), r = cadd(b, d), t = csub(b, d);
+  a = cadd(p, r);
+  c = csub(p, r);
+  b = make_float2(fmaf(-s, t.y, q.x), fmaf(s, t.x, q.y));
+  d = make_float2(fmaf(s, t.y, q.x), fmaf(-s, t.x, q.y));
+}
+
+// In-register DFT of N = 8 or 16 points: v[k] = sum_j v[j] W_N^(jk), W_N =
+// exp(sgn 2 pi i / N).  Radix 4 (8 = 2 x 4, 16 = 4 x 4) with the quarter and
+// eighth turns written out: 56 and 162 instructions, where a radix-2 recursion
+// that multiplies by every twiddle takes 96 and 256.
 template <int N>
 __device__ __forceinline__ void fft_reg(float2 *v, float sgn) {
-  if constexpr (N == 1) {
-    return;
+  static_assert(N == 8 || N == 16, "8 or 16 points");
+  if constexpr (N == 8) {
+    float2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
+    float2 o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
+    fft_reg4(e0, e1, e2, e3, sgn);
+    fft_reg4(o0, o1, o2, o3, sgn);
+    o1 = rot45(o1, sgn);
+    o2 = make_float2(-sgn * o2.y, sgn * o2.x);
+    o3 = rot135(o3, sgn);
+    v[0] = cadd(e0, o0);
+    v[4] = csub(e0, o0);
+    v[1] = cadd(e1, o1);
+    v[5] = csub(e1, o1);
+    v[2] = cadd(e2, o2);
+    v[6] = csub(e2, o2);
+    v[3] = cadd(e3, o3);
+    v[7] = csub(e3, o3);
   } else {
-    float2 e[N / 2], o[N / 2];
+    // cos, sin of an eighth of pi
+    constexpr float C = 0.92387953251128674f, S = 0.38268343236508978f;
+    // column b holds elements 4 a + b; after its DFT entry k1 takes W16^(b k1)
 #pragma unroll
-    for (int k = 0; k < N / 2; k++) {
-      e[k] = v[2 * k];
-      o[k] = v[2 * k + 1];
-    }
-    fft_reg<N / 2>(e, sgn);
-    fft_reg<N / 2>(o, sgn);
+    for (int b = 0; b < 4; b++) fft_reg4(v[b], v[4 + b], v[8 + b], v[12 + b], sgn);
+    v[5] = cmul(v[5], make_float2(C, sgn * S));
+    v[9] = rot45(v[9], sgn);
+    v[13] = cmul(v[13], make_float2(S, sgn * C));
+    v[6] = rot45(v[6], sgn);
+    v[10] = make_float2(-sgn * v[10].y, sgn * v[10].x);
+    v[14] = rot135(v[14], sgn);
+    v[7] = cmul(v[7], make_float2(S, sgn * C));
+    v[11] = rot135(v[11], sgn);
+    v[15] = cmul(v[15], make_float2(-C, -sgn * S));
+    // row k1 (v[4 k1 ..]) gives outputs k1 + 4 k2
 #pragma unroll
-    for (int k = 0; k < N / 2; k++) {
-      const int m = k * (16 / N);  // W_N^k = W_16^(k * 16 / N)
-      const float2 w = make_float2(C16[m], sgn * S16[m]);
-      const float2 t = cmul(o[k], w);
-      v[k] = cadd(e[k], t);
-      v[k + N / 2] = csub(e[k], t);
-    }
+    for (int k = 0; k < 4; k++) fft_reg4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3], sgn);
+    // transpose to natural order
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = i + 1; j < 4; j++) {
+        const float2 t = v[4 * i + j];
+        v[4 * i + j] = v[4 * j + i];
+        v[4 * j + i] = t;
+      }
   }
 }
 

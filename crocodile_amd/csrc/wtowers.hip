@@ -850,20 +850,33 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
             if (c == 0) s_pos[i] = r.x;
           }
           __syncthreads();
-          for (int i = 0; i < m; i++) {
-            const uint32_t pos = s_pos[i];
-            const int wx = (int)(pos & 0xffffu), dy = y - (int)(pos >> 16);
-            if ((unsigned)dy < (unsigned)S) {
-              const float2 kyv = s_ky[i][dy];
-              const int o = (j2 - wx) & 7;  // first window column of this thread
-              float2 *cell = lds + y * FP + wx + o;
-              if (o < S) {
-                const float2 t = cmul(s_vk[i][o], kyv);
-                cell[0] = make_float2(cell[0].x + neg * t.x, cell[0].y + neg * t.y);
-              }
-              if (o + 8 < S) {
-                const float2 t = cmul(s_vk[i][o + 8], kyv);
-                cell[8] = make_float2(cell[8].x + neg * t.x, cell[8].y + neg * t.y);
+          // the wavefront's eight rows meet few of the staged windows (18 % at
+          // S = 16): each lane tests one record, and the wavefront walks the
+          // set bits of the ballot, in record order, with the corner in a
+          // scalar register
+          {
+            const int lane = tid & 63;
+            const int r8 = 8 * __builtin_amdgcn_readfirstlane(tid >> 6);  // its first row
+            const uint32_t mypos = s_pos[min(lane, m - 1)];
+            const int wy0 = (int)(mypos >> 16);
+            unsigned long long hits = __ballot(lane < m && wy0 < r8 + 8 && wy0 + S > r8);
+            while (hits) {
+              const int i = __ffsll((long long)hits) - 1;
+              hits &= hits - 1;
+              const uint32_t pos = __builtin_amdgcn_readlane(mypos, i);
+              const int wx = (int)(pos & 0xffffu), dy = y - (int)(pos >> 16);
+              if ((unsigned)dy < (unsigned)S) {
+                const float2 kyv = s_ky[i][dy];
+                const int o = (j2 - wx) & 7;  // first window column of this thread
+                float2 *cell = lds + y * FP + wx + o;
+                if (o < S) {
+                  const float2 t = cmul(s_vk[i][o], kyv);
+                  cell[0] = make_float2(cell[0].x + neg * t.x, cell[0].y + neg * t.y);
+                }
+                if (o + 8 < S) {
+                  const float2 t = cmul(s_vk[i][o + 8], kyv);
+                  cell[8] = make_float2(cell[8].x + neg * t.x, cell[8].y + neg * t.y);
+                }
               }
             }
           }
