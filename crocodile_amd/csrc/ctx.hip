@@ -197,7 +197,10 @@ extern "C" int croc_last_kernel_ms(croc_ctx *ctx, float *grid_ms,
   return CROC_OK;
 }
 
-void tap_timer_reset(croc_ctx *ctx, int dir) { ctx->tev_n[dir] = 0; }
+void tap_timer_reset(croc_ctx *ctx, int dir) {
+  ctx->tev_n[dir] = 0;
+  ctx->tap_is_ev[dir] = false;
+}
 
 int tap_timer_begin(croc_ctx *ctx, int dir) {
   std::vector<hipEvent_t> &v = ctx->tev[dir];
@@ -223,6 +226,11 @@ extern "C" int croc_last_tap_kernel_ms(croc_ctx *ctx, float *grid_ms, int *grid_
   CROC_HIP(hipSetDevice(ctx->device));
   float tot[2] = {0.f, 0.f};
   for (int d = 0; d < 2; d++) {
+    if (ctx->tap_is_ev[d]) {
+      CROC_HIP(hipEventSynchronize(ctx->ev[2 * d + 1]));
+      CROC_HIP(hipEventElapsedTime(&tot[d], ctx->ev[2 * d], ctx->ev[2 * d + 1]));
+      continue;
+    }
     for (int k = 0; k < ctx->tev_n[d]; k++) {
       float ms = 0.f;
       CROC_HIP(hipEventSynchronize(ctx->tev[d][2 * (size_t)k + 1]));
@@ -231,9 +239,9 @@ extern "C" int croc_last_tap_kernel_ms(croc_ctx *ctx, float *grid_ms, int *grid_
     }
   }
   if (grid_ms) *grid_ms = tot[0];
-  if (grid_launches) *grid_launches = ctx->tev_n[0];
+  if (grid_launches) *grid_launches = ctx->tap_is_ev[0] ? 1 : ctx->tev_n[0];
   if (degrid_ms) *degrid_ms = tot[1];
-  if (degrid_launches) *degrid_launches = ctx->tev_n[1];
+  if (degrid_launches) *degrid_launches = ctx->tap_is_ev[1] ? 1 : ctx->tev_n[1];
   return CROC_OK;
 }
 

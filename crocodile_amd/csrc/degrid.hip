@@ -149,6 +149,10 @@ extern "C" int croc_convdegrid(croc_ctx *ctx, const void *grid, int N,
 
   BinArgs a{N, uvw, nv, stride, lam, Q, nplanes, plane_s, plane_off, separable,
             plane_mode, vplane, wstep, wbin0, max_support};
+  if (direct_degrid_wins(a, max_support)) {
+    if ((rc = bin_check(ctx, a, max_support))) return rc;
+    return direct_degrid(ctx, a, grid, vis_out, kern);
+  }
   BinPlan plan;
   rc = bin_visibilities(ctx, ctx->ws, a, max_support, ITEMS_BY_GROUP, &plan);
   if (rc) return rc;

@@ -69,6 +69,7 @@ enum WsSlot {
   WS_BL,        // baseline layout: flattened coordinates, planes, visibilities
   WS_BL_BANK,   // baseline layout: kernel-bank plane tables, unit kernel, FP32 table
   WS_BL_WIN,    // baseline layout: per-subgrid windows of a batched streamer call
+  WS_DIRECT,    // direct path: status, scale state, partial maxima
   WS_COUNT
 };
 
@@ -101,6 +102,11 @@ struct croc_ctx {
   // read it has been waited for)
   void *stage = nullptr;
   size_t stage_size = 0;
+  // direct path: its status word (WS_DIRECT) is known to be zero
+  bool direct_clean = false;
+  // the last gridding (0) / degridding (1) call's tap kernel is the one
+  // launch between ev[2 dir] and ev[2 dir + 1]
+  bool tap_is_ev[2] = {false, false};
   int num_cu = 256;
   int tile = 0;     // 0: automatic
   int chunk = 512;  // visibilities per work item
@@ -392,7 +398,39 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
+// Fixed-point scale exponent e of gridding: (nv + 1) * c * 2^e < 2^62 (no sum
+// overflows) and c * 2^e < 2^50 (the range fixed2 needs), c = 2 * max|v| *
+// max|k|^(1 or 2) bounding one contribution; mv, mk the largest component
+// magnitudes of the visibilities and the kernel bank.
+__device__ __forceinline__ int fixed_exponent(float mv, float mk, int64_t nv, int separable) {
+  double k = (double)mk;
+  if (separable) k = k * k * 2.0;  // product of two table entries
+  const double one = 2.0 * (double)mv * k;
+  const double bound = one * (double)(nv + 1);
+  int e = 40;
+  if (bound > 0.0 && isfinite(bound)) {
+    int ex, ex1;
+    frexp(bound, &ex);  // bound < 2^ex
+    frexp(one, &ex1);   // one < 2^ex1
+    e = min(61 - ex, 50 - ex1);
+  }
+  return max(-1000, min(e, 1000));
+}
+
 int choose_tile(croc_ctx *ctx, int max_support);
+// Sizes and geometry of a gridding / degridding call (CROC_EINVAL).
+int bin_check(croc_ctx *ctx, const BinArgs &a, int max_support);
+// Direct path (direct.hip): small one-shot calls without binning.
+bool direct_grid_wins(const BinArgs &a, int max_support);
+bool direct_degrid_wins(const BinArgs &a, int max_support);
+int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern);
+int direct_degrid(croc_ctx *ctx, const BinArgs &a, const void *grid, void *vis_out,
+                  const void *kern);
+// NaN into the cells that a non-finite visibility (flags bit 0) or kernel
+// value (bit 1) reaches (grid.hip).
+int grid_mark_nonfinite(croc_ctx *ctx, void *grid, int N, const uint4 *rec, int64_t nv,
+                        const void *vis, const void *kern, int separable,
+                        const uint32_t *flags);
 int choose_region(int T, int max_support);
 // Tile-kernel launches on binned visibilities (grid.hip, degrid.hip); they
 // read no status.  Record w holds the visibility's index into vis.
@@ -412,6 +450,8 @@ int bin_visibilities(croc_ctx *ctx, WsSet &set, const BinArgs &a, int max_suppor
 int read_status(croc_ctx *ctx, const BinPlan &plan);
 int persistent_blocks(croc_ctx *ctx, int per_cu);
 int zero_u32_async(croc_ctx *ctx, uint32_t *p, int64_t n);
+// Two ranges cleared by one launch.
+int zero2_u32_async(croc_ctx *ctx, uint32_t *p, int64_t n, uint32_t *q, int64_t m);
 
 // Batched centred 2D DFT (dft.hip): out[oi(b)] = out_scale * D in[ii(b)] D
 // with optional per-pixel modulation exp(i sign k[b] phi[pixel]) of the

@@ -353,8 +353,17 @@ class KernelBank:
         self.kern = kern
         self.plane_off_h = numpy.array(plane_off, dtype=numpy.int64)
         self.plane_s_h = numpy.array(plane_s, dtype=numpy.int32)
-        self.plane_off = torch.as_tensor(self.plane_off_h, device=dev)
-        self.plane_s = torch.as_tensor(self.plane_s_h, device=dev)
+        n = len(self.plane_s_h)
+        if n == 1 and self.plane_off_h[0] == 0:
+            # the single-table calls' bank: two fills instead of copies that wait
+            self.plane_off = torch.zeros(1, dtype=torch.int64, device=dev)
+            self.plane_s = torch.full((1,), int(self.plane_s_h[0]), dtype=torch.int32, device=dev)
+        else:  # both tables in one upload
+            both = numpy.zeros(n + (n + 1) // 2, dtype=numpy.int64)
+            both[:n] = self.plane_off_h
+            both[n:].view(numpy.int32)[:n] = self.plane_s_h
+            both_d = torch.as_tensor(both, device=dev)
+            self.plane_off, self.plane_s = both_d[:n], both_d[n:].view(torch.int32)[:n]
         self.Q = int(Q)
         self.separable = bool(separable)
         self.nplanes = len(self.plane_s_h)
