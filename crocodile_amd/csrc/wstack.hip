@@ -14,7 +14,7 @@
 // exp(i pi N / 2) is 1), so no shift pass touches the stack.
 #include <algorithm>
 
-#include "internal.h"
+#include "fft128.h"
 
 namespace {
 
@@ -163,7 +163,254 @@ __global__ __launch_bounds__(512) void k_wplane_sums(const double *__restrict__ 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The planes' inverse transforms for power-of-two grids, the sum over planes
+// fused into the column pass.
+//
+// A transform of N = 2^L points is Stockham radix-8 passes and a last pass of
+// radix N / 8^k, eight elements per thread in registers (j + s N / 8, s = 0 ..
+// 7, before and after), exchanged through LDS between passes; N / 8 threads to
+// a line.  Rows are transformed in place (k_wst_rows).  The column pass
+// (k_wst_cols_add) holds a tile of columns, walks the planes, and leaves
+// each plane's transform in registers, where the Fresnel phase is applied and
+// the sum kept in FP64: the transformed planes never go back to memory.
+// Memory traffic is one read and one write of the stack for the rows and
+// one read for the columns, against four of each (two transposes), a copy
+// and k_wstack_add's read; that traffic is the bound.  Twiddles come from an
+// FP64-rounded table in LDS, so rounding matches a plain FP32 FFT.
+//
+// wstack2048 (65 planes): 960 + 1230 us, where the library transform, its
+// input copy and k_wstack_add took 4.67 ms.
+template <int L>
+struct WstFft {
+  static constexpr int N = 1 << L;
+  static constexpr int T = N / 8;               // threads per line
+  static constexpr int FULL = (L - 1) / 3;      // radix-8 passes before the last
+  static constexpr int NS = 1 << (3 * FULL);    // points already combined
+  static constexpr int RL = N / NS;             // last radix: 2, 4 or 8
+  static_assert(RL == 2 || RL == 4 || RL == 8, "last radix");
+};
+
+// v[r] twiddled by W_N^(e r), r = 1 .. R - 1 (inverse sign).
+template <int R>
+__device__ __forceinline__ void wst_twiddle(float2 *v, int stride, const float2 *tw, int e) {
+#pragma unroll
+  for (int r = 1; r < R; r++) v[r * stride] = cmul(v[r * stride], tw[e * r]);
+}
+
+// One line's transform: v holds elements j + s N / 8 and receives the
+// outputs of the same indices.  at(i) is the LDS slot of element i; barriers
+// are the workgroup's (every thread takes part).
+template <int L, class At>
+__device__ __forceinline__ void wst_line(float2 (&v)[8], int j, float2 *lds, const float2 *tw,
+                                         At at) {
+  using F = WstFft<L>;
+  constexpr float sgn = 1.0f;
+  int ns = 1;
+#pragma unroll
+  for (int p = 0; p < F::FULL; p++) {
+    const int k = j & (ns - 1);
+    if (p) wst_twiddle<8>(v, 1, tw, k * (F::N / (8 * ns)));
+    fft_reg<8>(v, sgn);
+    const int d = (j - k) * 8 + k;
+    __syncthreads();  // the previous pass's reads are done
+#pragma unroll
+    for (int r = 0; r < 8; r++) lds[at(d + r * ns)] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = lds[at(j + s * F::T)];
+    ns *= 8;
+  }
+  // last pass: outputs fall on the elements read
+  constexpr int U = 8 / F::RL;
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    wst_twiddle<F::RL>(v + u, U, tw, j + u * F::T);
+    if constexpr (F::RL == 8) {
+      fft_reg<8>(v, sgn);
+    } else if constexpr (F::RL == 4) {
+      fft_reg4(v[u], v[u + U], v[u + 2 * U], v[u + 3 * U], sgn);
+    } else {
+      const float2 a = v[u], b = v[u + U];
+      v[u] = cadd(a, b);
+      v[u + U] = csub(a, b);
+    }
+  }
+}
+
+__global__ void k_wst_twiddles(int N, float2 *__restrict__ tw) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= N) return;
+  double s, c;
+  sincospi(2.0 * (double)k / (double)N, &s, &c);
+  tw[k] = make_float2((float)c, (float)s);
+}
+
+// Rows in place: persistent workgroups, 4096 / N rows (512 threads) at a
+// time, the next rows loaded during the current ones' passes.
+constexpr int WST_ROW_NT = 512;
+template <int L>
+__global__ __launch_bounds__(WST_ROW_NT) void k_wst_rows(float2 *__restrict__ stack,
+                                                        int64_t nrows,
+                                                        const float2 *__restrict__ twg) {
+  using F = WstFft<L>;
+  constexpr int LINES = WST_ROW_NT / F::T;
+  __shared__ float2 lds[LINES * F::N + LINES * F::N / 32];
+  __shared__ float2 tw[F::N];
+  const int tid = threadIdx.x, line = tid / F::T, j = tid % F::T;
+  for (int k = tid; k < F::N; k += WST_ROW_NT) tw[k] = twg[k];
+  auto at = [&](int i) {
+    const int e = line * F::N + i;
+    return e + (e >> 5);
+  };
+  const int64_t ngroups = nrows / LINES;  // N is a multiple of LINES
+  float2 nxt[8];
+  int64_t g = blockIdx.x;
+  auto load = [&](int64_t q) {
+    const float2 *row = stack + (q * LINES + line) * F::N + j;
+#pragma unroll
+    for (int s = 0; s < 8; s++) nxt[s] = row[s * F::T];
+  };
+  if (g < ngroups) load(g);
+  __syncthreads();  // table written
+  for (; g < ngroups; g += gridDim.x) {
+    float2 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = nxt[s];
+    if (g + gridDim.x < ngroups) load(g + gridDim.x);
+    wst_line<L>(v, j, lds, tw, at);
+    float2 *row = stack + (g * LINES + line) * F::N + j;
+#pragma unroll
+    for (int s = 0; s < 8; s++) row[s * F::T] = v[s];
+  }
+}
+
+// Columns of every plane and the phase-weighted sum: image[y][x] += sign
+// sum_p column transform of plane p at (y, x) times exp(-2 pi i midw[p] n1),
+// as k_wstack_add.  8192 / N columns (1024 threads) per workgroup and the
+// planes [p0, p1) of its plane group (blockIdx.y); workgroups of one XCD take
+// neighbouring columns, which share cache lines.  With one plane group the sum
+// is added without atomics.
+constexpr int WST_COL_NT = 1024;
+template <int L>
+__global__ __launch_bounds__(WST_COL_NT) void k_wst_cols_add(
+    double2 *__restrict__ image, const float2 *__restrict__ stack, int P, double theta,
+    const double *__restrict__ midw, const float2 *__restrict__ twg) {
+#pragma clang fp contract(off)
+  using F = WstFft<L>;
+  constexpr int TC = WST_COL_NT / F::T;  // columns of the tile
+  constexpr int E = TC * F::N;
+  __shared__ float2 lds[E + E / 8];
+  __shared__ float2 tw[F::N];
+  const int tid = threadIdx.x, c = tid % TC, j = tid / TC;
+  for (int k = tid; k < F::N; k += WST_COL_NT) tw[k] = twg[k];
+  constexpr int TILES = F::N / TC;
+  const int b = blockIdx.x;
+  const int tile = TILES % XCD_QUEUES == 0 ? (b % XCD_QUEUES) * (TILES / XCD_QUEUES) + b / XCD_QUEUES
+                                           : b;
+  const int x = tile * TC + c;
+  const int p0 = (int)((int64_t)P * blockIdx.y / gridDim.y);
+  const int p1 = (int)((int64_t)P * (blockIdx.y + 1) / gridDim.y);
+  auto at = [&](int i) {
+    const int e = i * TC + c;
+    return e + 4 * (e >> 5);
+  };
+  const int64_t NN = (int64_t)F::N * F::N;
+  const double l = theta * ((double)(x - F::N / 2) / (double)F::N);
+  double n1[8];
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int y = j + s * F::T;
+    const double m = theta * ((double)(y - F::N / 2) / (double)F::N);
+    n1[s] = 1.0 - sqrt(1.0 - (l * l + m * m));
+  }
+  double ax[8], ay[8];
+#pragma unroll
+  for (int s = 0; s < 8; s++) ax[s] = ay[s] = 0.0;
+  float2 nxt[8];
+  auto load = [&](int p) {
+    const float2 *col = stack + p * NN + (int64_t)j * F::N + x;
+#pragma unroll
+    for (int s = 0; s < 8; s++) nxt[s] = col[(int64_t)s * F::T * F::N];
+  };
+  if (p0 < p1) load(p0);
+  __syncthreads();  // table written
+  for (int p = p0; p < p1; p++) {
+    float2 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = nxt[s];
+    if (p + 1 < p1) load(p + 1);
+    wst_line<L>(v, j, lds, tw, at);
+    const double mw = midw[p];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      // turns reduced in FP64, the hardware sine and cosine of turns (1.24e-7
+      // largest absolute error), products and sum in FP64
+      const double t = mw * n1[s];
+      const float f = (float)(t - rint(t));
+      const double cs = (double)__builtin_amdgcn_cosf(f), sn = (double)__builtin_amdgcn_sinf(f);
+      const double vx = (double)v[s].x, vy = (double)v[s].y;
+      ax[s] = fma(vx, cs, fma(vy, sn, ax[s]));
+      ay[s] = fma(vy, cs, fma(-vx, sn, ay[s]));
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int y = j + s * F::T;
+    const double sg = ((x + y) & 1) ? -1.0 : 1.0;
+    double2 *o = image + (int64_t)y * F::N + x;
+    if (gridDim.y == 1) {
+      const double2 i = *o;
+      *o = make_double2(i.x + sg * ax[s], i.y + sg * ay[s]);
+    } else {
+      unsafeAtomicAdd(&o->x, sg * ax[s]);
+      unsafeAtomicAdd(&o->y, sg * ay[s]);
+    }
+  }
+}
+
+template <int L>
+void wst_image(croc_ctx *ctx, double2 *image, float2 *stack, int P, double theta,
+               const double *midw, float2 *tw) {
+  constexpr int N = 1 << L;
+  hipStream_t s = ctx->stream;
+  k_wst_twiddles<<<(N + 255) / 256, 256, 0, s>>>(N, tw);
+  const int64_t nrows = (int64_t)P * N, groups = nrows * N / (8 * WST_ROW_NT);
+  k_wst_rows<L><<<(unsigned)std::min<int64_t>(groups, 3 * (int64_t)ctx->num_cu), WST_ROW_NT, 0,
+                  s>>>(stack, nrows, tw);
+  // plane groups where the columns alone would not fill the chip
+  const int tiles = N / (8 * WST_COL_NT / N);
+  const int ng = std::max(1, std::min(P, 2 * ctx->num_cu / tiles));
+  k_wst_cols_add<L><<<dim3((unsigned)tiles, (unsigned)ng), WST_COL_NT, 0, s>>>(
+      image, stack, P, theta, midw, tw);
+}
+
 }  // namespace
+
+extern "C" int croc_wstack_image(croc_ctx *ctx, void *image, void *stack, int P, int N,
+                                 double theta, const double *midw) {
+  int rc = ctx_enter(ctx);
+  if (rc) return rc;
+  CROC_REQUIRE(image && stack && midw && P >= 1 && theta > 0, CROC_EINVAL, "bad arguments");
+  CROC_REQUIRE(N == 256 || N == 512 || N == 1024 || N == 2048, CROC_EINVAL,
+               "N must be 256, 512, 1024 or 2048");
+  const double c = theta * ((double)(0 - N / 2) / (double)N);
+  CROC_REQUIRE(c * c + c * c < 1.0, CROC_EDOMAIN, "Error in image coordinate system");
+  float2 *tw = (float2 *)ws_get(ctx, WS_TMP, sizeof(float2) * N);
+  if (!tw) return CROC_ENOMEM;
+  double2 *im = (double2 *)image;
+  float2 *st = (float2 *)stack;
+  if (N == 256)
+    wst_image<8>(ctx, im, st, P, theta, midw, tw);
+  else if (N == 512)
+    wst_image<9>(ctx, im, st, P, theta, midw, tw);
+  else if (N == 1024)
+    wst_image<10>(ctx, im, st, P, theta, midw, tw);
+  else
+    wst_image<11>(ctx, im, st, P, theta, midw, tw);
+  CROC_HIP(hipGetLastError());
+  return CROC_OK;
+}
 
 extern "C" int croc_wplane_sums(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride,
                                 double wstep, int64_t plane0, int ntab, int64_t *count,

@@ -1411,12 +1411,17 @@ def w_stacking_imaging(theta, lam, uvw, src, vis, wstep, max_stack_bytes=4 << 30
         _lib.check(L.croc_wstack_grid(_lib.ctx(), _lib.ptr(st), P, N, _lib.ptr(uv),
                                       uv.shape[0], uv.shape[1], float(lam), float(wstep),
                                       lo, ntab, _lib.ptr(slot_of), _lib.ptr(vt), centred))
+        mw = midw[b0:b0 + P].contiguous()
+        if N in (256, 512, 1024, 2048):
+            # power-of-two grids: transforms with the plane sum fused
+            _lib.check(L.croc_wstack_image(_lib.ctx(), _lib.ptr(image), _lib.ptr(st), P, N,
+                                           float(theta), _lib.ptr(mw)))
+            continue
         if centred:
             img = torch.fft.ifftn(st, dim=(-2, -1), norm='forward')
         else:
             img = torch.fft.fftshift(torch.fft.ifftn(torch.fft.ifftshift(st, dim=(-2, -1)),
                                                      dim=(-2, -1), norm='forward'), dim=(-2, -1))
-        mw = midw[b0:b0 + P].contiguous()
         _lib.check(L.croc_wstack_add(_lib.ctx(), _lib.ptr(image), _lib.ptr(img), P, N,
                                      float(theta), _lib.ptr(mw), centred))
         del img

@@ -232,6 +232,12 @@ int croc_wstack_grid(croc_ctx *ctx, void *stack, int P, int N, const double *uvw
  * cell 10).  A plane outside the table is CROC_EPLANE. */
 int croc_wplane_sums(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride,
                      double wstep, int64_t plane0, int ntab, int64_t *count, double *sum);
+/* croc_wstack_image: the inverse transforms of the stack's planes and
+ * croc_wstack_add (centred) in one: image += N^2 times the phase-weighted sum
+ * of the planes' inverse transforms, for N = 256, 512, 1024 or 2048.  The stack
+ * is overwritten. */
+int croc_wstack_image(croc_ctx *ctx, void *image, void *stack, int P, int N,
+                      double theta, const double *midw);
 int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
                     double theta, const double *midw, int centred);
 

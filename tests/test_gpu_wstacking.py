@@ -149,3 +149,30 @@ def test_plane_sums(gpu, ntab, nv, stride):
     if ntab > 1 and t.max() == ntab - 1:
         with pytest.raises(ValueError):
             _lib.check(call(ntab - 1))
+
+
+@pytest.mark.parametrize('N,P', [(256, 1), (256, 7), (512, 3), (1024, 2), (2048, 1)])
+def test_power_of_two_transforms(gpu, N, P):
+    """croc_wstack_image against FP64 FFTs of the same stack, every last-pass
+    radix, added to a non-zero image.  Bound: 4 log2(N) roundings of 2^-24 on
+    each of the two passes, relative to the sum of the planes' RMS."""
+    from crocodile_amd import _lib
+    g = torch.Generator(device='cuda').manual_seed(N + P)
+    theta = 0.3
+    st = torch.randn((P, N, N), generator=g, device='cuda', dtype=torch.complex64)
+    midw = torch.linspace(-300.0, 410.0, P, device='cuda', dtype=torch.float64)
+    x = (torch.arange(N, device='cuda', dtype=torch.float64) - N // 2) / N * theta
+    n1 = 1 - torch.sqrt(1 - x[None, :] ** 2 - x[:, None] ** 2)
+    i = torch.arange(N, device='cuda')
+    sign = (1 - 2 * ((i[:, None] + i[None, :]) % 2)).to(torch.float64)
+    base = torch.randn((N, N), generator=g, device='cuda', dtype=torch.complex128)
+    ref = base.clone()
+    for p in range(P):
+        ph = -2 * numpy.pi * midw[p] * n1
+        ref += (torch.fft.ifftn(st[p].to(torch.complex128), norm='forward') * sign
+                * torch.polar(torch.ones_like(ph), ph))
+    img = base.clone()
+    _lib.check(_lib.load().croc_wstack_image(_lib.ctx(), _lib.ptr(img), _lib.ptr(st.clone()), P, N,
+                                             theta, _lib.ptr(midw)))
+    err = (img - ref).abs().pow(2).mean().sqrt()
+    assert float(err / (ref - base).abs().pow(2).mean().sqrt()) < 8 * numpy.log2(N) * 2.0 ** -24
