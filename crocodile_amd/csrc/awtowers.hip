@@ -25,7 +25,10 @@
 // of the inverse transform and k_awt_place the output sign of the forward
 // one.
 #include <algorithm>
+#include <climits>
 #include <vector>
+
+#include <hipcub/hipcub.hpp>
 
 #include "internal.h"
 
@@ -133,6 +136,119 @@ __global__ void k_awt_apply(float2 *__restrict__ bins, int c0,
   *o = b;
 }
 
+// Chunk numbers ub, vb = floor(u theta / chunk + 0.5) and w-plane rint(w /
+// wstep) of every visibility, their ranges, and the antenna indices checked.
+__global__ void k_awt_bins(const double *__restrict__ uvw, int64_t nv, int64_t stride,
+                           double theta, double wstep, int chunk,
+                           const int64_t *__restrict__ src, int64_t nant, int4 *__restrict__ bin,
+                           int *__restrict__ range, uint32_t *__restrict__ status) {
+#pragma clang fp contract(off)
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  int v[3] = {INT_MAX, INT_MAX, INT_MAX}, w[3] = {INT_MIN, INT_MIN, INT_MIN};
+  if (i < nv) {
+    const double a = floor(uvw[i * stride] * theta / (double)chunk + 0.5);
+    const double b = floor(uvw[i * stride + 1] * theta / (double)chunk + 0.5);
+    const double c = rint(uvw[i * stride + 2] / wstep);
+    const int64_t s1 = src[2 * i], s2 = src[2 * i + 1];
+    if (!(fabs(a) < 0x1p30 && fabs(b) < 0x1p30 && fabs(c) < 0x1p30)) {
+      atomicOr(status, (uint32_t)ST_DOMAIN);
+    } else if (s1 < 0 || s2 < 0 || s1 >= nant || s2 >= nant) {
+      atomicOr(status, (uint32_t)ST_PLANE);
+    } else {
+      v[0] = w[0] = (int)a;
+      v[1] = w[1] = (int)b;
+      v[2] = w[2] = (int)c;
+      bin[i] = make_int4((int)a, (int)b, (int)c, 0);
+    }
+  }
+  __shared__ int s_lo[3], s_hi[3];
+  if (threadIdx.x < 3) {
+    s_lo[threadIdx.x] = INT_MAX;
+    s_hi[threadIdx.x] = INT_MIN;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      v[k] = min(v[k], __shfl_xor(v[k], off, 64));
+      w[k] = max(w[k], __shfl_xor(w[k], off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&s_lo[k], v[k]);
+      atomicMax(&s_hi[k], w[k]);
+    }
+  }
+  barrier_after_lds_atomics();
+  if (threadIdx.x < 3 && s_lo[threadIdx.x] <= s_hi[threadIdx.x]) {
+    atomicMin(&range[threadIdx.x], s_lo[threadIdx.x]);
+    atomicMax(&range[3 + threadIdx.x], s_hi[threadIdx.x]);
+  }
+}
+
+__global__ void k_awt_range_init(int *range, uint32_t *status) {
+  if (threadIdx.x < 3) range[threadIdx.x] = INT_MAX;
+  else if (threadIdx.x < 6) range[threadIdx.x] = INT_MIN;
+  if (threadIdx.x == 6) *status = 0u;
+}
+
+struct AwtRange {
+  int ub, vb, wp;      // lowest
+  int64_t nvb, P, nant;
+};
+
+// Group key (chunk, plane, antenna pair) and index of every visibility.
+__global__ void k_awt_keys(const int4 *__restrict__ bin, const int64_t *__restrict__ src,
+                           int64_t nv, AwtRange r, uint64_t *__restrict__ key,
+                           int32_t *__restrict__ idx) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nv) return;
+  const int4 b = bin[i];
+  const uint64_t cid = (uint64_t)(b.x - r.ub) * r.nvb + (uint64_t)(b.y - r.vb);
+  key[i] = ((cid * r.P + (uint64_t)(b.z - r.wp)) * r.nant + (uint64_t)src[2 * i]) * r.nant +
+           (uint64_t)src[2 * i + 1];
+  idx[i] = (int32_t)i;
+}
+
+// Per group its plane and antennas, per run its chunk key; vstart's end.
+__global__ void k_awt_groups(const uint64_t *__restrict__ gkey, int ng, int64_t nv, AwtRange r,
+                             int32_t *__restrict__ gwp, int32_t *__restrict__ ga1,
+                             int32_t *__restrict__ ga2, uint64_t *__restrict__ gcid,
+                             int32_t *__restrict__ vstart) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g == 0) vstart[ng] = (int32_t)nv;
+  if (g >= ng) return;
+  uint64_t k = gkey[g];
+  ga2[g] = (int32_t)(k % r.nant);
+  k /= r.nant;
+  ga1[g] = (int32_t)(k % r.nant);
+  k /= r.nant;
+  gwp[g] = (int32_t)(k % r.P) + r.wp;
+  gcid[g] = k / r.P;
+}
+
+// Sorted visibility v: its group (the last start <= v) and its coordinates
+// relative to the group's chunk middle and plane.
+__global__ void k_awt_rel(const double *__restrict__ uvw, int64_t nv, int64_t stride,
+                          const int32_t *__restrict__ order, const int4 *__restrict__ bin,
+                          const int32_t *__restrict__ vstart, int ng, double theta, double wstep,
+                          int chunk, int32_t *__restrict__ gid, double *__restrict__ rel) {
+#pragma clang fp contract(off)
+  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= nv) return;
+  int lo = 0, hi = ng - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (vstart[mid] <= v) lo = mid; else hi = mid - 1;
+  }
+  gid[v] = lo;
+  const int64_t i = order[v];
+  const int4 b = bin[i];
+  rel[3 * v] = uvw[i * stride] - (double)chunk * (double)b.x / theta;
+  rel[3 * v + 1] = uvw[i * stride + 1] - (double)chunk * (double)b.y / theta;
+  rel[3 * v + 2] = uvw[i * stride + 2] - (double)b.z * wstep;
+}
+
 // Window corner and sub-offsets {xs, ys, xf, yf} of every visibility on the M
 // grid, as k_awt_pregrid places it.
 __global__ void k_awt_locate(const double *__restrict__ rel, int64_t nv, double lam_sub, int M,
@@ -172,7 +288,8 @@ __global__ void k_awt_locate(const double *__restrict__ rel, int64_t nv, double 
 // looked up in an FP64-rounded table, so the vectors carry FP32 rounding of
 // K terms only.  awtowers1800 (6991 groups, 12636 visibilities): 312 us in
 // place of 6.1 ms (clear, pre-grid, transform and its copies, apply); bound by
-// the LDS reads of the vectors (5 per 4 pixels and visibility).
+// latency, a segment's groups following one another with their screens' reads
+// (16-byte reads of Y, or 8 to 32 vectors staged at a time, change nothing).
 //
 // The vectors are centred, so the images carry the centring sign
 // (-1)^(x + y) that the pre-grids' uncentred transforms leave out (the input
@@ -183,7 +300,7 @@ __device__ __forceinline__ float chunk_window(const float *__restrict__ win, int
 }
 
 constexpr int AWD_T = 32;    // tile edge (pixels)
-constexpr int AWD_NT = 256;  // threads: column tid % 32, rows tid / 32 + 8 q
+constexpr int AWD_NT = 256;  // threads: column tid % 32, rows 4 (tid / 32) + q
 constexpr int AWD_VB = 16;   // visibilities whose vectors are staged at a time
 constexpr int AWD_MAX_M = 4096;  // twiddle table in LDS: 8 M bytes
 
@@ -196,7 +313,7 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
     const float *__restrict__ win, const double *__restrict__ turns,
     const float *__restrict__ lmag) {
   extern __shared__ float2 s_tw[];                // [M]
-  __shared__ float2 s_xy[AWD_VB][2 * AWD_T];      // X (first AWD_T), then v Y
+  __shared__ __align__(16) float2 s_xy[AWD_VB][2 * AWD_T];  // X (first AWD_T), then v Y
   const int tid = threadIdx.x, M = 2 * S, SS = S * S;
   for (int k = tid; k < M; k += AWD_NT) {
     double s, c;
@@ -214,7 +331,7 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
   bool in[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const int y = ty0 + ly + 8 * q;
+    const int y = ty0 + 4 * ly + q;
     in[q] = x < S && y < S;
     pix[q] = in[q] ? y * S + x : 0;  // pixel 0 stands in (never written)
     tw[q] = turns[pix[q]];
@@ -299,9 +416,12 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
         screens();
       }
       const float2 X = s_xy[k][lx];
+      const float4 *Y4 = (const float4 *)&s_xy[k][AWD_T + 4 * ly];
+      const float4 ya = Y4[0], yb = Y4[1];
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const float2 Y = s_xy[k][AWD_T + ly + 8 * q];
+        const float4 y2 = q < 2 ? ya : yb;
+        const float2 Y = q % 2 ? make_float2(y2.z, y2.w) : make_float2(y2.x, y2.y);
         ix[q] = fmaf(X.x, Y.x, fmaf(-X.y, Y.y, ix[q]));
         iy[q] = fmaf(X.x, Y.y, fmaf(X.y, Y.x, iy[q]));
       }
@@ -400,6 +520,99 @@ extern "C" int croc_awt_apply(croc_ctx *ctx, void *bins, int c0, int nc, const v
                                              start, gwp, ga1, ga2,
                                              (const float2 *)ascreen, win, turns, lmag);
   CROC_HIP(hipGetLastError());
+  return CROC_OK;
+}
+
+extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride,
+                               double theta, double wstep, int chunk, const int64_t *src,
+                               int64_t nant, int32_t *order, int32_t *vstart, int32_t *gid,
+                               double *rel, int32_t *gwp, int32_t *ga1, int32_t *ga2,
+                               int64_t *ngroups, int64_t *nchunks, int64_t *cstart,
+                               int32_t *cub, int32_t *cvb) {
+  int rc = ctx_enter(ctx);
+  if (rc) return rc;
+  CROC_REQUIRE(nv >= 1 && nv < (int64_t)INT32_MAX && stride >= 3 && theta > 0 && wstep > 0 &&
+                   chunk >= 1 && nant >= 1,
+               CROC_EINVAL, "bad arguments");
+  CROC_REQUIRE(uvw && src && order && vstart && gid && rel && gwp && ga1 && ga2 && ngroups &&
+                   nchunks && cstart && cub && cvb,
+               CROC_EINVAL, "null array");
+  const size_t n = (size_t)nv;
+  hipStream_t s = ctx->stream;
+  uint64_t *key = nullptr, *skey = nullptr, *gkey = nullptr;
+  int32_t *idx = nullptr, *count = nullptr;
+  size_t t_sort = 0, t_rle = 0, t_scan = 0;
+  CROC_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t_sort, key, skey, idx, order, (int)n, 0,
+                                              64, s));
+  CROC_HIP(hipcub::DeviceRunLengthEncode::Encode(nullptr, t_rle, skey, gkey, count,
+                                                 (int32_t *)nullptr, (int)n, s));
+  CROC_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, t_scan, count, vstart, (int)n, s));
+  const size_t tb = std::max(t_sort, std::max(t_rle, t_scan));
+  char *w = (char *)ws_get(ctx, WS_SORT, 512 + n * (16 + 3 * 8 + 2 * 4) + tb + 256);
+  int *small = (int *)ws_get(ctx, WS_SMALL, 256);
+  uint64_t *h = (uint64_t *)host_stage(ctx, sizeof(uint64_t) * n + 256);
+  if (!w || !small || !h) return CROC_ENOMEM;
+  int4 *bin = (int4 *)w;
+  key = (uint64_t *)(bin + n);
+  skey = key + n;
+  gkey = skey + n;
+  idx = (int32_t *)(gkey + n);
+  count = idx + n;
+  void *temp = (void *)(((uintptr_t)(count + n) + 255) & ~(uintptr_t)255);
+  uint32_t *st = (uint32_t *)small;
+  int *range = small + 8, *nruns = small + 16;
+  const unsigned nb = (unsigned)((nv + 255) / 256);
+  k_awt_range_init<<<1, 64, 0, s>>>(range, st);
+  k_awt_bins<<<nb, 256, 0, s>>>(uvw, nv, stride, theta, wstep, chunk, src, nant, bin, range, st);
+  CROC_HIP(hipGetLastError());
+  CROC_HIP(hipMemcpyAsync(h, small, 128, hipMemcpyDeviceToHost, s));
+  CROC_HIP(hipStreamSynchronize(s));
+  {
+    const uint32_t bits = *(const uint32_t *)h;
+    if (bits & ST_PLANE) {
+      croc_set_error("antenna index outside the A-screens");
+      return CROC_EPLANE;
+    }
+    if ((rc = croc_status_to_code(bits))) return rc;
+  }
+  const int *hr = (const int *)h + 8;
+  AwtRange r{hr[0], hr[1], hr[2], (int64_t)hr[4] - hr[1] + 1, (int64_t)hr[5] - hr[2] + 1, nant};
+  const double keys = ((double)hr[3] - hr[0] + 1) * (double)r.nvb * (double)r.P * (double)nant *
+                      (double)nant;
+  CROC_REQUIRE(keys < 0x1p62, CROC_EINVAL,
+               "too many (chunk, w-plane, antenna pair) groups; increase wstep");
+  int end_bit = 1;
+  while (end_bit < 62 && ldexp(1.0, end_bit) < keys) end_bit++;
+  k_awt_keys<<<nb, 256, 0, s>>>(bin, src, nv, r, key, idx);
+  size_t t = tb;
+  CROC_HIP(hipcub::DeviceRadixSort::SortPairs(temp, t, key, skey, idx, order, (int)n, 0, end_bit,
+                                              s));
+  t = tb;
+  CROC_HIP(hipcub::DeviceRunLengthEncode::Encode(temp, t, skey, gkey, count, nruns, (int)n, s));
+  CROC_HIP(hipMemcpyAsync(h, nruns, sizeof(int), hipMemcpyDeviceToHost, s));
+  CROC_HIP(hipStreamSynchronize(s));
+  const int ng = *(const int *)h;
+  t = tb;
+  CROC_HIP(hipcub::DeviceScan::ExclusiveSum(temp, t, count, vstart, ng, s));
+  uint64_t *gcid = key;  // the unsorted keys are no longer needed
+  k_awt_groups<<<(unsigned)((ng + 255) / 256), 256, 0, s>>>(gkey, ng, nv, r, gwp, ga1, ga2, gcid,
+                                                            vstart);
+  k_awt_rel<<<nb, 256, 0, s>>>(uvw, nv, stride, order, bin, vstart, ng, theta, wstep, chunk, gid,
+                               rel);
+  CROC_HIP(hipGetLastError());
+  CROC_HIP(hipMemcpyAsync(h, gcid, sizeof(uint64_t) * ng, hipMemcpyDeviceToHost, s));
+  CROC_HIP(hipStreamSynchronize(s));
+  int64_t nc = 0;
+  for (int g = 0; g < ng; g++) {
+    if (g == 0 || h[g] != h[g - 1]) {
+      cub[nc] = (int32_t)(h[g] / (uint64_t)r.nvb) + r.ub;
+      cvb[nc] = (int32_t)(h[g] % (uint64_t)r.nvb) + r.vb;
+      cstart[nc++] = g;
+    }
+  }
+  cstart[nc] = ng;
+  *ngroups = ng;
+  *nchunks = nc;
   return CROC_OK;
 }
 

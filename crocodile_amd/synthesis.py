@@ -1605,51 +1605,45 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     grid = torch.zeros((N, N), dtype=torch.complex64, device=dev)
     if nv == 0:
         return _out(grid, like_torch)
-    st = _dev(src, torch.int64).reshape(nv, -1)[:, :2]
+    st = _dev(src, torch.int64).reshape(nv, -1)[:, :2].contiguous()
     at = _dev(aimage, torch.complex64)
     nant = at.shape[0]
     if tuple(at.shape[1:]) != (S, S):
         raise ValueError('aimage must be [nant, subgrid_size, subgrid_size]')
-    if bool(((st < 0) | (st >= nant)).any()):
-        raise IndexError('antenna index outside the A-screens')
     gcf = _dev(aa_gcf, torch.complex64)
     if gcf.ndim != 2:
         raise ValueError('aa_gcf must be a separable [Q, K] table')
     Q, K = int(gcf.shape[0]), int(gcf.shape[1])
-    chunk = S - margin
-    wp = torch.round(uv[:, 2] / float(wstep)).to(torch.int64)
-    ub = torch.floor(uv[:, 0] * theta / chunk + 0.5).to(torch.int64)
-    vb = torch.floor(uv[:, 1] * theta / chunk + 0.5).to(torch.int64)
-    lo = torch.stack([wp.min(), ub.min(), vb.min()]).cpu().tolist()
-    hi = torch.stack([wp.max(), ub.max(), vb.max()]).cpu().tolist()
-    P, nub, nvb = (hi[k] - lo[k] + 1 for k in range(3))
-    cid = (ub - lo[1]) * nvb + (vb - lo[2])
-    key = ((cid * P + (wp - lo[0])) * nant + st[:, 0]) * nant + st[:, 1]
-    key, order = torch.sort(key, stable=True)
-    gkey, gcount = torch.unique_consecutive(key, return_counts=True)
-    G = gkey.shape[0]
-    ga2 = (gkey % nant).to(torch.int32)
-    ga1 = ((gkey // nant) % nant).to(torch.int32)
-    gwp_rel = (gkey // (nant * nant)) % P
-    gcid = gkey // (nant * nant * P)
-    gwp = gwp_rel + lo[0]
-    # chunks in key order, and each group's chunk slot
-    ccid, ccount = torch.unique_consecutive(gcid, return_counts=True)
-    C = ccid.shape[0]
-    gchunk = torch.repeat_interleave(torch.arange(C, device=dev), ccount)
-    ccid_h = ccid.cpu().numpy()
-    uv_mid, corner = _awt_chunks(theta, lam, S, margin, ccid_h // nvb + lo[1],
-                                 ccid_h % nvb + lo[2])
-    mid_g = torch.cat([torch.as_tensor(uv_mid, device=dev)[gchunk],
-                       (gwp.to(torch.float64) * float(wstep))[:, None]], 1)
-    gid = torch.repeat_interleave(torch.arange(G, device=dev, dtype=torch.int32), gcount)
-    rel = (uv[order, :3] - mid_g[gid.long()]).contiguous()
-    vc = _dev(vis, torch.complex128).reshape(-1)[order]
+    vis_t = _dev(vis, torch.complex128 if dl != 0 or dm != 0 else torch.complex64).reshape(-1)
+    if vis_t.shape[0] < nv:
+        raise ValueError('fewer visibilities than coordinates')
+    # groups sorted by (chunk, plane, antenna pair), on the device
+    ints = torch.empty((6, nv + 1), dtype=torch.int32, device=dev)
+    order, vstart32, gid, gwp32, ga1, ga2 = ints.unbind(0)
+    rel = torch.empty((nv, 3), dtype=torch.float64, device=dev)
+    cstart_h = numpy.empty(nv + 1, dtype=numpy.int64)
+    cub, cvb = numpy.empty((2, nv), dtype=numpy.int32)
+    ng, nc = ctypes.c_int64(), ctypes.c_int64()
+    rc = _lib.load().croc_awt_groups(
+        _lib.ctx(), _lib.ptr(uv), nv, uv.shape[1], float(theta), float(wstep), S - margin,
+        _lib.ptr(st), nant, _lib.ptr(order), _lib.ptr(vstart32), _lib.ptr(gid), _lib.ptr(rel),
+        _lib.ptr(gwp32), _lib.ptr(ga1), _lib.ptr(ga2), ctypes.byref(ng), ctypes.byref(nc),
+        cstart_h.ctypes.data_as(ctypes.c_void_p), cub.ctypes.data_as(ctypes.c_void_p),
+        cvb.ctypes.data_as(ctypes.c_void_p))
+    if rc == _lib.EPLANE:
+        raise IndexError('antenna index outside the A-screens')
+    _lib.check(rc)
+    G, C = ng.value, nc.value
+    cstart_h = cstart_h[:C + 1]
+    _, corner = _awt_chunks(theta, lam, S, margin, cub[:C], cvb[:C])
     if dl != 0 or dm != 0:
+        vc = vis_t.index_select(0, order[:nv])
         vc = vc / w_kernel_function(torch.tensor(float(dl), dtype=torch.float64, device=dev),
                                     torch.tensor(float(dm), dtype=torch.float64, device=dev),
                                     rel[:, 2])
-    vt = vc.to(torch.complex64).contiguous()
+        vt = vc.to(torch.complex64).contiguous()
+    else:
+        vt = vis_t.index_select(0, order[:nv])
     lam_sub = S / theta
     L = _lib.load()
     # image-space tables of the sub-grid; the window carries the inverse
@@ -1661,11 +1655,6 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     wk = _dev(wkern, torch.complex128)
     turns = (torch.angle(wk) / (2 * math.pi)).contiguous()
     lmag = torch.log2(torch.abs(wk)).to(torch.float32).contiguous()
-    # group ranges: visibility offsets and chunk offsets
-    vstart = torch.zeros(G + 1, dtype=torch.int64, device=dev)
-    vstart[1:] = torch.cumsum(gcount, 0)
-    cstart_h = numpy.concatenate([[0], numpy.cumsum(ccount.cpu().numpy())]).astype(numpy.int64)
-    gwp32 = gwp.to(torch.int32).contiguous()
     # Groups of few visibilities are summed directly (croc_awt_direct): ~15 ns
     # per visibility, where the pre-grids cost ~1 us per (2S)^2 grid and
     # 5 ns per visibility.  Measured with the awtowers1800 tracks repeated:
@@ -1675,7 +1664,6 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     # visibility per AWT_DIRECT_CELLS pre-grid cells.
     if nv * AWT_DIRECT_CELLS <= G * M * M and M <= 4096:
         bins = torch.empty((C, S, S), dtype=torch.complex64, device=dev)
-        vstart32 = vstart.to(torch.int32)
         _lib.check(L.croc_awt_direct(
             _lib.ctx(), _lib.ptr(bins), C, S, _lib.ptr(rel), nv, float(lam_sub), Q, K,
             _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(vstart32),
@@ -1683,8 +1671,8 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
             _lib.ptr(ga2), _lib.ptr(at), _lib.ptr(win), _lib.ptr(turns), _lib.ptr(lmag),
             min(int(max_stack_bytes), 1 << 30)))
     else:
-        bins = _awt_bins_fft(rel, vt, gid, vstart.cpu().numpy(), cstart_h, gwp32, ga1, ga2, S,
-                             lam_sub, gcf, at, win, turns, lmag, max_stack_bytes)
+        bins = _awt_bins_fft(rel, vt, gid, vstart32[:G + 1].cpu().numpy(), cstart_h, gwp32, ga1,
+                             ga2, S, lam_sub, gcf, at, win, turns, lmag, max_stack_bytes)
     fb = torch.fft.fftn(bins, dim=(-2, -1))
     corner_t = torch.as_tensor(corner.astype(numpy.int32), device=dev).contiguous()
     for c0 in range(0, C, 65535):

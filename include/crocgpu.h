@@ -248,6 +248,14 @@ int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
  * pair); gid[v] is visibility v's group, rel its [nv][3] coordinates
  * relative to its group's (u_mid, v_mid, wp * wstep).
  *
+ * croc_awt_groups sorts visibilities by group: chunk (ub, vb) = floor((u, v)
+ * theta / chunk + 0.5), w-plane round-half-even(w / wstep), antenna pair src
+ * (int64 [nv][2], indices outside [0, nant) are CROC_EPLANE).  Device outputs:
+ * order [nv] (sorted -> input index, stable), vstart [nv + 1] (first
+ * visibility of each group, and the end), gid and rel [nv] (sorted order), gwp /
+ * ga1 / ga2 [nv] (per group).  Host outputs: the group and chunk counts, cstart
+ * [nv + 1] (first group of each chunk, and the end), cub / cvb [nv].
+ *
  * croc_awt_pregrid grids visibilities [v0, v1) onto stack[gid - g0]
  * ([G][M][M] cf32, M = 2 * subgrid_size) with the separable cf32 table gcf
  * [Q][K] at p = rel / lam_sub (synthesis.py:451-481's convgrid, frac_coord
@@ -273,6 +281,12 @@ int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
  *
  * croc_awt_place adds (-1)^(x+y) bins[c] (forward transformed) into grid
  * ([N][N] cf32) at corner[c] = (x0, y0), clipped at the grid's edges. */
+int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride,
+                    double theta, double wstep, int chunk, const int64_t *src,
+                    int64_t nant, int32_t *order, int32_t *vstart, int32_t *gid,
+                    double *rel, int32_t *gwp, int32_t *ga1, int32_t *ga2,
+                    int64_t *ngroups, int64_t *nchunks, int64_t *cstart, int32_t *cub,
+                    int32_t *cvb);
 int croc_awt_pregrid(croc_ctx *ctx, void *stack, int M, const double *rel, int64_t v0,
                      int64_t v1, double lam_sub, int Q, int K, const void *gcf,
                      const void *vis, const int32_t *gid, int32_t g0, int check_only);
