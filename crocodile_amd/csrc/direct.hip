@@ -129,7 +129,7 @@ __global__ __launch_bounds__(DIR_NT) void k_direct_grid(
 // host words.
 __global__ __launch_bounds__(DIR_NT) void k_direct_finish(
     float2 *__restrict__ grid, const longlong2 *__restrict__ acc, int64_t cells, int nparts,
-    DirectState *__restrict__ st, uint32_t *__restrict__ host) {
+    DirectState *__restrict__ st, uint32_t *__restrict__ host, float sign) {
   __shared__ uint32_t s[DIR_WAVES];
   const uint32_t status = st->status;
   if (blockIdx.x == 0) {
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(DIR_NT) void k_direct_finish(
     if (c.x | c.y) {
       float2 g = grid[i];
       g.x += (float)((double)c.x * inv);
-      g.y += (float)((double)c.y * inv);
+      g.y = sign * (sign * g.y + (float)((double)c.y * inv));
       grid[i] = g;
     }
   }
@@ -248,7 +248,8 @@ bool direct_degrid_wins(const BinArgs &a, int max_support) {
          a.nv <= DIRECT_DEGRID_TAPS / ((int64_t)max_support * max_support);
 }
 
-int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern) {
+int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern,
+                float sign) {
   const int64_t cells = (int64_t)a.N * a.N;
   ulonglong2 *acc = (ulonglong2 *)ws_get(ctx, WS_ACC, sizeof(ulonglong2) * cells);
   if (!acc) return CROC_ENOMEM;
@@ -274,7 +275,8 @@ int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, co
   CROC_HIP(hipEventRecord(ctx->ev[1], s));
   ctx->ev_grid = ctx->tap_is_ev[0] = true;
   k_direct_finish<<<(unsigned)std::min<int64_t>((cells + DIR_NT - 1) / DIR_NT, 8192), DIR_NT, 0,
-                    s>>>((float2 *)grid, (const longlong2 *)acc, cells, DIR_PARTS, st, host);
+                    s>>>((float2 *)grid, (const longlong2 *)acc, cells, DIR_PARTS, st, host,
+                          sign);
   CROC_HIP(hipGetLastError());
   if ((rc = direct_end(ctx, host))) return rc;
   if (host[1])  // non-finite values: their cells, on the stream

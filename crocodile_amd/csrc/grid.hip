@@ -250,9 +250,11 @@ __global__ void k_grid_lists(const int4 *__restrict__ items, const uint32_t *__r
 }
 
 // grid[c] += acc[c] / 2^e, clearing nothing (the workspace is zeroed per call).
+// sign = -1 adds the conjugate, rounded as on a grid conjugated before and
+// after (two passes over the grid that this saves).
 __global__ void k_grid_finish(float2 *__restrict__ grid,
                               const long long *__restrict__ acc, int64_t n,
-                              const ScaleState *__restrict__ st) {
+                              const ScaleState *__restrict__ st, float sign) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const long long re = acc[2 * i], im = acc[2 * i + 1];
@@ -260,7 +262,7 @@ __global__ void k_grid_finish(float2 *__restrict__ grid,
     const double s = st->inv_scale;
     float2 g = grid[i];
     g.x += (float)((double)re * s);
-    g.y += (float)((double)im * s);
+    g.y = sign * (sign * g.y + (float)((double)im * s));
     grid[i] = g;
   }
 }
@@ -303,7 +305,7 @@ __global__ void k_grid_nonfinite(float2 *__restrict__ grid, int N,
 // status read.
 int grid_binned(croc_ctx *ctx, const BinPlan &plan, void *grid, int N,
                 int64_t nv, const void *vis, const void *kern, int Q, int separable,
-                int nplanes, const int64_t *plane_off, const int32_t *plane_s) {
+                int nplanes, const int64_t *plane_off, const int32_t *plane_s, float sign) {
   int rc;
   const int64_t cells = (int64_t)N * N;
   unsigned long long *acc =
@@ -361,7 +363,7 @@ int grid_binned(croc_ctx *ctx, const BinPlan &plan, void *grid, int N,
   CROC_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
   ctx->ev_grid = true;
   k_grid_finish<<<(unsigned)((cells + 255) / 256), 256, 0, ctx->stream>>>(
-      (float2 *)grid, (const long long *)acc, cells, st);
+      (float2 *)grid, (const long long *)acc, cells, st, sign);
   return grid_mark_nonfinite(ctx, grid, N, plan.rec, nv, vis, kern, separable, &st->nonfinite);
 }
 
@@ -396,16 +398,22 @@ extern "C" int croc_convgrid(croc_ctx *ctx, void *grid, int N,
 
   BinArgs a{N, uvw, nv, stride, lam, Q, nplanes, plane_s, plane_off, separable,
             plane_mode, vplane, wstep, wbin0, max_support};
+  return convgrid_run(ctx, a, max_support, grid, vis, kern, 1.0f);
+}
+
+int convgrid_run(croc_ctx *ctx, const BinArgs &a, int max_support, void *grid, const void *vis,
+                 const void *kern, float sign) {
+  int rc;
   if (direct_grid_wins(a, max_support)) {
     if ((rc = bin_check(ctx, a, max_support))) return rc;
-    return direct_grid(ctx, a, grid, vis, kern);
+    return direct_grid(ctx, a, grid, vis, kern, sign);
   }
   BinPlan plan;
   // both lists: the per-XCD one carries the dense tiles (see k_grid_tiles)
   rc = bin_visibilities(ctx, ctx->ws, a, max_support, ITEMS_BY_TILE | ITEMS_BY_GROUP, &plan);
   if (rc) return rc;
-  rc = grid_binned(ctx, plan, grid, N, nv, vis, kern, Q, separable, nplanes,
-                   plane_off, plane_s);
+  rc = grid_binned(ctx, plan, grid, a.N, a.nv, vis, kern, a.Q, a.separable, a.nplanes,
+                   a.plane_off, a.plane_s, sign);
   if (rc) return rc;
   rc = read_status(ctx, plan);
   return rc;

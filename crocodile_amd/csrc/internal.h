@@ -423,7 +423,9 @@ int bin_check(croc_ctx *ctx, const BinArgs &a, int max_support);
 // Direct path (direct.hip): small one-shot calls without binning.
 bool direct_grid_wins(const BinArgs &a, int max_support);
 bool direct_degrid_wins(const BinArgs &a, int max_support);
-int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern);
+// sign: as grid_binned's.
+int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern,
+                float sign);
 int direct_degrid(croc_ctx *ctx, const BinArgs &a, const void *grid, void *vis_out,
                   const void *kern);
 // NaN into the cells that a non-finite visibility (flags bit 0) or kernel
@@ -433,10 +435,14 @@ int grid_mark_nonfinite(croc_ctx *ctx, void *grid, int N, const uint4 *rec, int6
                         const uint32_t *flags);
 int choose_region(int T, int max_support);
 // Tile-kernel launches on binned visibilities (grid.hip, degrid.hip); they
-// read no status.  Record w holds the visibility's index into vis.
+// read no status.  Record w holds the visibility's index into vis.  sign = -1
+// adds the conjugate of the gridded values (+1: the values).
 int grid_binned(croc_ctx *ctx, const BinPlan &plan, void *grid, int N,
                 int64_t nv, const void *vis, const void *kern, int Q, int separable,
-                int nplanes, const int64_t *plane_off, const int32_t *plane_s);
+                int nplanes, const int64_t *plane_off, const int32_t *plane_s, float sign);
+// One gridding call on checked arguments, direct or by tiles (grid.hip).
+int convgrid_run(croc_ctx *ctx, const BinArgs &a, int max_support, void *grid, const void *vis,
+                 const void *kern, float sign);
 int degrid_binned(croc_ctx *ctx, const BinPlan &plan, const void *grid, int N, void *vis_out,
                   const void *kern, int separable);
 // Work-item lists (bit mask): ITEMS_BY_TILE cuts each tile's records (all

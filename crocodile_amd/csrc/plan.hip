@@ -99,7 +99,7 @@ extern "C" int croc_convgrid_plan(croc_ctx *ctx, croc_plan *plan, void *grid,
   rc = zero_u32_async(ctx, plan->bp.qhead, XCD_QUEUES + 1);  // work queues restart
   if (rc) return rc;
   return grid_binned(ctx, plan->bp, grid, plan->N, plan->nv, vis, kern, plan->Q,
-                     plan->separable, plan->nplanes, plan->plane_off, plan->plane_s);
+                     plan->separable, plan->nplanes, plan->plane_off, plan->plane_s, 1.0f);
 }
 
 extern "C" int croc_convdegrid_plan(croc_ctx *ctx, croc_plan *plan, const void *grid,

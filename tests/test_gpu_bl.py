@@ -383,3 +383,27 @@ def test_degrid_boxes_and_groups_agree(gpu, S):
     size = B.degrid_conv_uv(numpy.abs(g.real) + numpy.abs(g.imag) + 0j, theta, uv,
                             numpy.abs(kern)).real
     assert (numpy.abs(ordered - ref) <= (S * S + 8) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize('nbl', [20, 600])  # direct path, tile path
+def test_grid_wprojection_adds_conjugate(gpu, nbl):
+    """w_project's conjugate is taken where the fixed-point sums are added, so a
+    grid that holds values gains exactly what a cleared one is given."""
+    print('case grid_wprojection conjugate', nbl, flush=True)
+    rng = numpy.random.default_rng(nbl)
+    N, theta, S, Q, P = 256, 0.02, 8, 4, 3
+    wk = c64(rng.normal(size=(P, Q, Q, S, S)) + 1j * rng.normal(size=(P, Q, Q, S, S)))
+    host, dev = make_set(rng, nbl, 20, 24, 9000.0, ragged=True)
+    assert (len(host.vis) * S * S <= 3 << 20) == (nbl == 20)
+    w = lam(host, 2)
+    w_min, w_step = w.min() + 5.0, (w.max() - w.min()) / (P - 1.5)
+    ref = numpy.zeros((N, N), dtype=complex)
+    B.grid_wprojection(ref, theta, host, wk, w_min, w_step)
+    wkd = BL.WKernelData(wk, w_min, w_step)
+    gd = torch.zeros((N, N), dtype=torch.complex64, device=gpu)
+    assert BL.grid_wprojection(gd, N, theta, dev, wkd) == len(host.vis) * 8 * S * S
+    assert_close(gd.cpu().numpy(), ref, what='grid_wprojection')
+    base = torch.as_tensor(c64(rng.normal(size=(N, N)) + 1j * rng.normal(size=(N, N)))).to(gd)
+    got = base.clone()
+    BL.grid_wprojection(got, N, theta, dev, wkd)
+    assert torch.equal(got, base + gd)
