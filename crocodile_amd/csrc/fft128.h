@@ -33,11 +33,40 @@ struct FModArgs {
 // error on [-1/2, 1/2], measured against FP64 over 2^20 points; a library
 // sincosf of the FP32 angle in radians is 2.1e-7 there and several times
 // the instructions).
-__device__ __forceinline__ float2 rotate(float2 v, double kf, double phi) {
+__device__ __forceinline__ float2 rotation(double kf, double phi) {  // {cos, sin}
   const double t = kf * phi * 0.15915494309189535;
   const float f = (float)(t - rint(t));
   const float s = __builtin_amdgcn_sinf(f), c = __builtin_amdgcn_cosf(f);
-  return make_float2(v.x * c - v.y * s, v.x * s + v.y * c);
+  return make_float2(c, s);
+}
+__device__ __forceinline__ float2 rotate_by(float2 v, float2 r) {
+  return make_float2(v.x * r.x - v.y * r.y, v.x * r.y + v.y * r.x);
+}
+__device__ __forceinline__ float2 rotate(float2 v, double kf, double phi) {
+  return rotate_by(v, rotation(kf, phi));
+}
+
+// The rotations of one w-plane, each taken once: phi depends on the pixel's
+// distances u, w from the middle row and column only, and not on their order
+// (to the bit: its l^2 + m^2 is formed symmetrically), so 2145 of the 16384
+// pixels' rotations differ.  Entry (hi, lo) = (max, min)(u, w), 0 <= lo <= hi
+// <= 64, sits at |hi - 32| ROT_P + (hi > 32 ? lo : 66 - lo): rows hi and
+// 64 - hi share a line, and with the odd pitch a half-wavefront along a row or
+// a column of pixels takes 1.6 passes over the banks on average.
+constexpr int ROT_P = 67;
+constexpr int ROT_N = 33 * ROT_P;
+
+__device__ __forceinline__ int rot_index(int y, int x) {
+  const int u = abs(x - FN / 2), w = abs(y - FN / 2);
+  const int hi = max(u, w), lo = min(u, w);
+  return abs(hi - 32) * ROT_P + (hi > 32 ? lo : 66 - lo);
+}
+
+// rot[e] = rotation(kf, phic[e]), by the whole workgroup; phic in the layout
+// above.
+__device__ __forceinline__ void rot_table(float2 *rot, const double *__restrict__ phic,
+                                          double kf) {
+  for (int e = threadIdx.x; e < ROT_N; e += FFT_NT) rot[e] = rotation(kf, phic[e]);
 }
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }

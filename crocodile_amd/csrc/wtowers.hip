@@ -781,7 +781,15 @@ constexpr int TW_STAGE = 64;
 //     its own row elements (row y, columns x = j2 mod 8: at most two per
 //     window) into the LDS sub-grid in record order,
 //       G[wy + dy][wx + dx] += (v kx[dx]) ky[dy]
-//     (the taps of synthesis.py:456), before the transform reads them.
+//     (the taps of synthesis.py:456), before the transform reads them.  The
+//     plane's rotations come from a table in LDS (phi: its layout) that takes
+//     the place of the staged rows; SMALL = false computes them per pixel
+//     (phi: by pixel): its registers hold the next job's rows, and with the
+//     table it spilled up to 55 of them (N = 2048, a million visibilities,
+//     two-dimensional kernel: 615 us per pixel, 702 with the table).
+// The table takes 2145 rotations per job in place of 16384 (FP64 reduction and
+// two quarter-rate sines each) and their angles' loads: N = 4096, 6.73 ms in
+// place of 7.05, N = 8192 2.06 in place of 2.18.
 template <bool SMALL>
 __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
     const int4 *__restrict__ runs, int nruns, const int32_t *__restrict__ jl,
@@ -792,7 +800,17 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
   constexpr int NS = SMALL ? TW_STAGE : 1;
   __shared__ float2 lds[FN * FP];
   __shared__ float2 tw[FN];
-  __shared__ float2 s_vk[NS][16], s_ky[NS][16];  // v kx and ky rows (zero beyond S)
+  // small jobs: v kx and ky rows (zero beyond S); then, read by the last
+  // column pass, the plane's rotations
+  union Stage {
+    struct {
+      float2 vk[NS][16], ky[NS][16];
+    } k;
+    float2 rot[SMALL ? ROT_N : 1];
+  };
+  __shared__ Stage s_stage;
+  auto &s_vk = s_stage.k.vk;
+  auto &s_ky = s_stage.k.ky;
   __shared__ uint32_t s_pos[NS];                 // window corners wx | wy << 16
   __shared__ int s_need[SMALL ? FN : 1];         // small jobs: rows holding taps,
   __shared__ int s_rows[SMALL ? FN : 1];         // listed in order
@@ -901,6 +919,7 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
         __syncthreads();
         nrows = s_nrows;
         rows_pass_a(lds, s_rows, nrows, twz, sgn);  // rows without taps stay zero
+        rot_table(s_stage.rot, phi, -(double)kw[job]);  // the staged rows are read
       } else {
         float2 v[16];
 #pragma unroll
@@ -951,8 +970,13 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
           int x, k1;
           cols_pass_b_item(r, x, k1);
           double ph[8];
+          if constexpr (!SMALL) {
 #pragma unroll
-          for (int k2 = 0; k2 < 8; k2++) ph[k2] = phi[zero + (k1 + 16 * k2) * FN + x];
+            for (int k2 = 0; k2 < 8; k2++) ph[k2] = phi[zero + (k1 + 16 * k2) * FN + x];
+          }
+          // the table positions computed here, not kept over the jobs (16
+          // registers, spilled): the wavefront's rows are uniform
+          const int xz = x + zero, kz = __builtin_amdgcn_readfirstlane(k1) + zero;
           float2 v[8];
           const float2 *p = lds + x + 8 * k1 * FP;
 #pragma unroll
@@ -961,7 +985,9 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_image_runs(
           const float sc = ((x + k1) & 1) ? -out_scale : out_scale;
 #pragma unroll
           for (int k2 = 0; k2 < 8; k2++) {
-            const float2 t = rotate(make_float2(v[k2].x * sc, v[k2].y * sc), kout, ph[k2]);
+            const float2 w = make_float2(v[k2].x * sc, v[k2].y * sc);
+            const float2 t = SMALL ? rotate_by(w, s_stage.rot[rot_index(kz + 16 * k2, xz)])
+                                   : rotate(w, kout, ph[k2]);
             acc[r][k2] = make_float2(acc[r][k2].x + t.x, acc[r][k2].y + t.y);
           }
         }
@@ -1197,19 +1223,23 @@ __device__ __forceinline__ void degrid_round16(const float2 *lds, int j0, int j1
 //      columns first, then the rows the item's windows cover (all rows
 //      when it holds more than FFT_NT visibilities); the chunk image's
 //      columns are read at each item (consecutive items mostly share it);
+//      the plane's 2145 different rotations are taken once, into an LDS table,
+//      instead of one per pixel with its angle read from memory (N = 8192:
+//      5.05 ms in place of 5.53, N = 4096: 5.54 in place of 6.94);
 //   2. the item's visibilities degridded from LDS, several lanes per
 //      visibility; the window lies inside the sub-grid (S <= margin,
 //      checked at binning).
 template <int SF>
 __global__ __launch_bounds__(FFT_NT) void k_tw_predict_sep(
     const int4 *__restrict__ items, const int32_t *__restrict__ roff, int nruns,
-    const float2 *__restrict__ cimg, const double *__restrict__ phi,
+    const float2 *__restrict__ cimg, const double *__restrict__ phic,
     const uint4 *__restrict__ rec, const float2 *__restrict__ kern, int S, int64_t tsize,
     float2 *__restrict__ vis_out, uint32_t *__restrict__ qc) {
   __shared__ float2 lds[FN * FP];
   __shared__ float2 tw[FN];
   __shared__ int s_need[FN];  // rows some window of the item covers
   __shared__ int s_rows[FN];  // those rows, ascending
+  __shared__ float2 s_rot[ROT_N];  // the item's plane's rotations
   __shared__ int s_nrows, s_run;
   const int tid = threadIdx.x;
   constexpr float sgn = -1.0f;  // forward transform
@@ -1233,14 +1263,10 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_predict_sep(
       const float2 *twz = tw + zero;
       {
         float2 v[16];
-        double ph[16];
         const float2 *col = cimg + (int64_t)it.x * SGN + c2 * FN + x;
-        const double *pcol = phi + zero + c2 * FN + x;
 #pragma unroll
-        for (int j1 = 0; j1 < 16; j1++) {
-          v[j1] = col[8 * j1 * FN];
-          ph[j1] = pcol[8 * j1 * FN];
-        }
+        for (int j1 = 0; j1 < 16; j1++) v[j1] = col[8 * j1 * FN];
+        rot_table(s_rot, phic, (double)it.y);  // last read before the row passes
         __syncthreads();  // tw written; the previous item's LDS reads done
         // the rows the item's windows cover (s_need was cleared after the
         // previous item's row passes)
@@ -1252,10 +1278,9 @@ __global__ __launch_bounds__(FFT_NT) void k_tw_predict_sep(
           for (int k = 0; k < S; k++) s_need[wy + k] = 1;
         }
         const float neg = ((x + c2) & 1) ? -1.0f : 1.0f;
-        const double kin = (double)it.y;
 #pragma unroll
         for (int j1 = 0; j1 < 16; j1++) {
-          const float2 t = rotate(v[j1], kin, ph[j1]);
+          const float2 t = rotate_by(v[j1], s_rot[rot_index(8 * j1 + c2, x)]);
           v[j1] = make_float2(neg * t.x, neg * t.y);
         }
         fft_reg<16>(v, sgn);
@@ -1438,6 +1463,26 @@ __global__ void k_tw_phi(double *phi, double theta, double wstep) {
   const double m = ((double)(y - SG / 2) / (double)SG) * theta;
   const double r2 = l * l + m * m;
   phi[i] = r2 < 1.0 ? 2.0 * M_PI * wstep * (1.0 - sqrt(1.0 - r2)) : 0.0;
+}
+
+// The same for the entries of a rotation table (fft128.h), zero where it has none.
+__global__ void k_tw_phi_table(double *phic, double theta, double wstep) {
+#pragma clang fp contract(off)
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= ROT_N) return;
+  const int row = e / ROT_P, col = e - row * ROT_P;
+  int hi = 32 + row, lo = col;
+  if (row == 0 || lo > hi) {
+    hi = 32 - row;
+    lo = 66 - col;
+  }
+  double phi = 0.0;
+  if (lo >= 0 && lo <= hi) {
+    const double l = ((double)hi / (double)SG) * theta, m = ((double)lo / (double)SG) * theta;
+    const double r2 = l * l + m * m;
+    if (r2 < 1.0) phi = 2.0 * M_PI * wstep * (1.0 - sqrt(1.0 - r2));
+  }
+  phic[e] = phi;
 }
 
 // Gridding schedule of a binning, made on the host once and kept on the
@@ -1936,7 +1981,7 @@ int tw_grid_run(croc_ctx *ctx, const Plan &p, void *grid, const void *kern, int 
   const bool mfma = !a.nearest && separable && a.S <= 16;
   CROC_REQUIRE(mfma ? p.gss_ready : p.gs_ready, CROC_EINVAL, "gridding schedule missing");
   const GridSched &gs = mfma ? p.gs_split : p.gs;
-  char *aux = (char *)ws_get(ctx, WS_SCALE, 256 + sizeof(double) * SGN +
+  char *aux = (char *)ws_get(ctx, WS_SCALE, 256 + sizeof(double) * (SGN + ROT_N) +
                                                 sizeof(uint32_t) * (2 * gs.batches.size() + 64) +
                                                 sizeof(uint32_t) * (size_t)a.ncx * a.ncx);
   const size_t cimg_bytes = sizeof(float2) * SGN * (size_t)a.ncx * a.ncx;
@@ -1944,8 +1989,8 @@ int tw_grid_run(croc_ctx *ctx, const Plan &p, void *grid, const void *kern, int 
       (float2 *)ws_get(ctx, WS_SUB, cimg_bytes + sizeof(float2) * SGN * (size_t)gs.max_slots);
   if (!aux || !stack) return CROC_ENOMEM;
   TwScale *fs = (TwScale *)aux;
-  double *phi = (double *)(aux + 256);
-  uint32_t *qc = (uint32_t *)(phi + SGN);  // part queues, then summing-run queues
+  double *phi = (double *)(aux + 256), *phic = phi + SGN;  // by pixel; rotation table's layout
+  uint32_t *qc = (uint32_t *)(phic + ROT_N);  // part queues, then summing-run queues
   uint32_t *cflag = qc + 2 * gs.batches.size() + 64;  // chunks to set non-finite
   float2 *cimg = stack, *sub = stack + (size_t)SGN * a.ncx * a.ncx;
   if ((rc = zero_u32_async(ctx, (uint32_t *)fs, sizeof(TwScale) / 4))) return rc;
@@ -1961,6 +2006,8 @@ int tw_grid_run(croc_ctx *ctx, const Plan &p, void *grid, const void *kern, int 
                                                                   ksplit);
   }
   k_tw_phi<<<SGN / 256, 256, 0, s>>>(phi, a.theta, a.wstep);
+  if (gs.small.nr)
+    k_tw_phi_table<<<(ROT_N + 255) / 256, 256, 0, s>>>(phic, a.theta, a.wstep);
   CROC_HIP(hipGetLastError());
   // zero the chunk images that will receive data
   k_tw_zero_chunks<<<dim3(16, (unsigned)p.chunks.size()), 256, 0, s>>>(gs.chunks, cimg);
@@ -1974,7 +2021,7 @@ int tw_grid_run(croc_ctx *ctx, const Plan &p, void *grid, const void *kern, int 
     // slots 0, 1, ... before the batches take the slots
     k_tw_image_runs<true><<<(unsigned)std::min<size_t>(gs.small.nr, (size_t)ctx->num_cu), FFT_NT,
                             0, s>>>(gs.runs + gs.small.r0, (int)gs.small.nr, gs.jl, gs.jslot,
-                                    gs.kw, phi, sub, cimg, qc + 2 * gs.batches.size(), p.jobs,
+                                    gs.kw, phic, sub, cimg, qc + 2 * gs.batches.size(), p.jobs,
                                     p.rec, p.svis, (const float2 *)kern, a.S, tsize);
     CROC_HIP(hipGetLastError());
     if (gs.small.nq) {
@@ -2086,10 +2133,13 @@ int tw_degrid_run(croc_ctx *ctx, const Plan &p, const void *grid, void *vis_out,
   float2 *stack = (float2 *)ws_get(
       ctx, WS_SUB, cimg_bytes + (sep16 ? 0 : sizeof(float2) * SGN * (size_t)ds.jb));
   if (!aux || !stack) return CROC_ENOMEM;
-  double *phi = (double *)(aux + 256);
+  double *phi = (double *)(aux + 256);  // sep16: in the rotation table's layout
   uint32_t *qc = (uint32_t *)(phi + SGN);  // a part queue per batch
   float2 *cimg = stack, *sub = stack + (size_t)SGN * a.ncx * a.ncx;
-  k_tw_phi<<<SGN / 256, 256, 0, s>>>(phi, a.theta, a.wstep);
+  if (sep16)
+    k_tw_phi_table<<<(ROT_N + 255) / 256, 256, 0, s>>>(phi, a.theta, a.wstep);
+  else
+    k_tw_phi<<<SGN / 256, 256, 0, s>>>(phi, a.theta, a.wstep);
   if ((rc = zero_u32_async(ctx, qc, (int64_t)ds.poff.size()))) return rc;
   dim3 g(16, (unsigned)p.chunks.size());
   CROC_HIP(hipEventRecord(ctx->ev[2], s));

@@ -9,7 +9,7 @@ from crocodile_amd import _lib
 from oracle import synthesis_ref as R
 from oracle import wtowers_ref as WT
 
-from test_gpu_core import assert_close
+from test_gpu_core import MAX_TOL, RMS_TOL, assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -256,3 +256,27 @@ def test_wtowers_job_size_bounds(gpu, support):
     assert_close(v, vref, what='w_towers_predict job size bounds S=%d' % support)
     plan = G.WTowersPlan(THETA, LAM, uvw, 40.0, SG, MARGIN, kv)
     assert (plan.imaging(vis, kv) == g).all() and (plan.predict(grid, kv) == v).all()
+
+
+@pytest.mark.parametrize('theta', [0.1, 1.5])
+@pytest.mark.parametrize('support', [5, 16])
+def test_wtowers_rotation_table_matches_per_pixel_phase(gpu, theta, support):
+    """A separable kernel takes each plane's rotations from a table over the
+    distances from the middle pixel, the outer product of the same kernel per
+    pixel.  theta = 1.5 reaches pixels beyond the horizon (no phase).  Both
+    are within assert_close of the exact result, so within twice that of each
+    other."""
+    print('case rotation table', theta, support, flush=True)
+    rng = numpy.random.default_rng(support)
+    lam, nv = 512 / theta, 3000  # jobs of few visibilities
+    r = 0.35 * lam * numpy.sqrt(rng.uniform(0, 1, nv))
+    ph = rng.uniform(0, 2 * numpy.pi, nv)
+    uvw = numpy.stack([r * numpy.cos(ph), r * numpy.sin(ph), rng.uniform(-90, 90, nv)], 1)
+    vis = rng.standard_normal(nv) + 1j * rng.standard_normal(nv)
+    sep = rng.standard_normal((4, support)) + 1j * rng.standard_normal((4, support))
+    two = sep[:, None, :, None] * sep[None, :, None, :]
+    grid = rng.standard_normal((512, 512)) + 1j * rng.standard_normal((512, 512))
+    out = [G.w_towers_imaging(theta, lam, uvw, None, vis, 3.0, SG, MARGIN, k) for k in (sep, two)]
+    assert_close(out[0], out[1], 2 * RMS_TOL, 2 * MAX_TOL, 'imaging')
+    out = [G.w_towers_predict(theta, lam, uvw, None, grid, 3.0, SG, MARGIN, k) for k in (sep, two)]
+    assert_close(out[0], out[1], 2 * RMS_TOL, 2 * MAX_TOL, 'predict')
