@@ -472,7 +472,7 @@ __global__ __launch_bounds__(TW_NT) void k_tw_grid_jobs_mfma(
   const unsigned long long lt = (1ull << lane) - 1ull;
   const float sk = unit_scale(__uint_as_float(fs->max_k_bits));
   const float sv = unit_scale(__uint_as_float(fs->max_vis_bits));
-  const float in_scale = sv * sk * sk, out_scale = 1.f / in_scale;
+  const float out_scale = 1.f / (sv * sk * sk);
   uint2 *ring = s_ring[wave];
   ring[lane] = make_uint2(0u, 0u);  // slots past the listed ones are read, then ignored
   ring[lane + 64] = make_uint2(0u, 0u);
@@ -596,16 +596,6 @@ __global__ __launch_bounds__(TW_NT) void k_tw_grid_jobs_mfma(
         const int by = blk >> 3, bx = blk & 7;
         const int r0 = 16 * by, c0 = 16 * bx;
         tw_floatx4 cr = {0.f, 0.f, 0.f, 0.f}, ci = {0.f, 0.f, 0.f, 0.f};
-        if (win) {
-          // later windows go on from the block's sum so far (the scale is a
-          // power of two): its loads overlap the listing
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const float2 old = out[(r0 + 4 * (lane >> 4) + q) * SG + c0 + m];
-            cr[q] = old.x * in_scale;
-            ci[q] = old.y * in_scale;
-          }
-        }
         uint32_t head = 0, tail = 0;
         // K-group of 32 listed visibilities starting at ring position h
         // (nvalid of them real, the rest zero)
@@ -688,7 +678,13 @@ __global__ __launch_bounds__(TW_NT) void k_tw_grid_jobs_mfma(
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           float2 *o = out + (r0 + 4 * (lane >> 4) + q) * SG + c0 + m;
-          *o = make_float2(cr[q] * out_scale, ci[q] * out_scale);
+          float2 val = make_float2(cr[q] * out_scale, ci[q] * out_scale);
+          if (win) {
+            const float2 old = *o;
+            val.x += old.x;
+            val.y += old.y;
+          }
+          *o = val;
         }
       }
       __syncthreads();  // the window's records are read; the next one rewrites them
