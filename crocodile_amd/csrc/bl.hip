@@ -14,6 +14,7 @@
 // does.
 #include <algorithm>
 
+#include "blbox.h"
 #include "internal.h"
 
 namespace {
@@ -389,7 +390,6 @@ __device__ __forceinline__ int wave_extreme(int v) {
 // L1 accesses (90 % of the cycles, ~18 per visibility, each row straddling
 // two 64-byte lines); from the LDS box 2.1
 // ms.
-constexpr int BL_BOX = 600;  // cells per wavefront: 19 KiB a workgroup
 typedef float bl_cell2 __attribute__((ext_vector_type(4), aligned(8)));  // two cells
 
 template <int G, int W>
@@ -459,8 +459,8 @@ __global__ __launch_bounds__(BL_NT) void k_bl_degrid(DegridArgs a) {
             ymin = wave_extreme<false>(mine ? y0 : INT32_MAX);
             bw = wave_extreme<true>(mine ? x0 : INT32_MIN) - xmin + S;
             bh = wave_extreme<true>(mine ? y0 : INT32_MIN) - ymin + S;
-            pitch = bw | 1;  // rows on different banks
-            return bh * pitch <= BL_BOX;
+            pitch = bl_box_pitch(bw);
+            return bl_box_fits(bw, bh);
           };
           if (!bounds()) {  // one dump of the batch, if it holds enough of it
             const int lead = __builtin_amdgcn_readlane(t, __ffsll((long long)left) - 1);

@@ -407,3 +407,27 @@ def test_grid_wprojection_adds_conjugate(gpu, nbl):
     got = base.clone()
     BL.grid_wprojection(got, N, theta, dev, wkd)
     assert torch.equal(got, base + gd)
+
+
+def test_degrid_windows_across_a_large_grid(gpu):
+    """Wavefronts whose windows span more cells than 2^31 (46400 a side): the
+    corners' visibilities taken in turn equal the same ones taken corner by
+    corner, bit for bit."""
+    print('case degrid_conv_uv N=46400', flush=True)
+    rng = numpy.random.default_rng(46)
+    N, theta, S, Q, n = 46400, 0.02, 8, 16, 64
+    gd = torch.zeros((N, N), dtype=torch.complex64, device=gpu)
+    patch, _ = rand_grid(rng, 64)
+    patch = torch.as_tensor(patch.astype(numpy.complex64)).cuda()
+    for ys in (slice(0, 64), slice(N - 64, N)):
+        for xs in (slice(0, 64), slice(N - 64, N)):
+            gd[ys, xs] = patch
+    lo, hi = -N // 2 + S // 2, N - N // 2 - (S - S // 2)
+    a, b = rng.uniform(0, 9, (2, 4, n))
+    u = numpy.where(numpy.array([0, 1, 0, 1])[:, None], hi - a, lo + a) / theta
+    v = numpy.where(numpy.array([0, 0, 1, 1])[:, None], hi - b, lo + b) / theta
+    k = BL.SepKernelData(rng.normal(size=(Q, S)))
+    by_corner = BL.degrid_conv_uv(gd, N, theta, u.ravel(), v.ravel(), k).cpu().numpy()
+    in_turn = BL.degrid_conv_uv(gd, N, theta, u.T.ravel(), v.T.ravel(), k).cpu().numpy()
+    assert (by_corner != 0).all()
+    assert_array_equal(in_turn.reshape(n, 4).T.ravel(), by_corner)
