@@ -1606,6 +1606,8 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     if nv == 0:
         return _out(grid, like_torch)
     st = _dev(src, torch.int64).reshape(nv, -1)[:, :2].contiguous()
+    if st.shape[1] < 2:  # the kernels read two indices per visibility
+        raise IndexError('src must hold an antenna pair per visibility')
     at = _dev(aimage, torch.complex64)
     nant = at.shape[0]
     if tuple(at.shape[1:]) != (S, S):

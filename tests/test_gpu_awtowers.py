@@ -97,6 +97,21 @@ def test_errors(gpu):
     assert empty.shape == (sc['N'], sc['N']) and not empty.any()
 
 
+@pytest.mark.parametrize('form', ['column', 'flat', 'empty'])
+def test_src_without_pairs(gpu, form):
+    """One antenna index per visibility, or none, is refused before the
+    device reads pairs."""
+    sc = scenario()
+    nv = len(sc['uvw'])
+    src = {'column': numpy.zeros((nv, 1), int), 'flat': numpy.zeros(nv, int),
+           'empty': numpy.zeros((nv, 0), int)}[form]
+    wk = R.w_kernel_function(sc['l'], sc['m'], 2.0)
+    with pytest.raises((IndexError, RuntimeError)):
+        G.aw_towers_imaging(sc['theta'], sc['lam'], sc['uvw'], src, sc['vis'], 2.0, sc['S'],
+                            sc['margin'], sc['aa_gcf'], sc['aa_sub'], sc['aa_sub2'],
+                            sc['aimage'], wk)
+
+
 @pytest.mark.parametrize('direct', [True, False])
 @pytest.mark.parametrize('S,margin,K,budget', [(32, 6, 6, 4 << 30),    # one pixel tile
                                                (34, 8, 5, 4 << 30),    # ragged tiles, odd support
