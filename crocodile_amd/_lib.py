@@ -65,6 +65,7 @@ SIGNATURES = {
     'croc_remap_coords': [_P, _P, _I64, _I64, _D, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     'croc_grid_nearest': [_P, _P, _I, _P, _I64, _I64, _D, _P],
     'croc_wstack_grid': [_P, _P, _I, _I, _P, _I64, _I64, _D, _D, _I64, _I, _P, _P, _I],
+    'croc_w_bins': [_P, _P, _I64, _I64, _D, _P],
     'croc_wplane_sums': [_P, _P, _I64, _I64, _D, _I64, _I, _P, _P],
     'croc_wstack_image': [_P, _P, _P, _I, _I, _D, _P],
     'croc_wstack_add': [_P, _P, _P, _I, _I, _D, _P, _I],

@@ -39,7 +39,7 @@ class WProjectionOperator:
         self.uvw = (uvw.to(dev, torch.float64) if isinstance(uvw, torch.Tensor)
                     else torch.as_tensor(numpy.asarray(uvw, dtype=numpy.float64), device=dev)
                     ).contiguous()
-        wb = torch.round(self.uvw[:, 2] / self.wstep).to(torch.int64)
+        wb = G._w_bins(self.uvw, self.wstep)
         self.wbin0, hi = int(wb.min()), int(wb.max())
         ws = [self.wstep * b for b in range(self.wbin0, hi + 1)]
         S = [support(w) if callable(support) else int(support) for w in ws]

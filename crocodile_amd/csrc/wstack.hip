@@ -112,6 +112,13 @@ __global__ void k_wstack_add(double2 *__restrict__ image,
   image[pix] = o;
 }
 
+__global__ void k_w_bins(const double *__restrict__ w, int64_t nv, int64_t stride, double wstep,
+                         int64_t *__restrict__ bin) {
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += step)
+    bin[i] = wbin_dev(w[i * stride], wstep);
+}
+
 // Visibility count and sum of w of every w-plane t = round-half-even(w /
 // wstep) - plane0, t < ntab: block-private histograms in LDS (sums by FP64 LDS
 // atomics), one global atomic per block and non-empty plane.  A plane outside
@@ -408,6 +415,19 @@ extern "C" int croc_wstack_image(croc_ctx *ctx, void *image, void *stack, int P,
     wst_image<10>(ctx, im, st, P, theta, midw, tw);
   else
     wst_image<11>(ctx, im, st, P, theta, midw, tw);
+  CROC_HIP(hipGetLastError());
+  return CROC_OK;
+}
+
+extern "C" int croc_w_bins(croc_ctx *ctx, const double *w, int64_t nv, int64_t stride,
+                           double wstep, int64_t *bin) {
+  int rc = ctx_enter(ctx);
+  if (rc) return rc;
+  CROC_REQUIRE(nv >= 0 && stride >= 1, CROC_EINVAL, "bad arguments");
+  if (nv == 0) return CROC_OK;
+  CROC_REQUIRE(w && bin, CROC_EINVAL, "null array");
+  const unsigned nb = (unsigned)std::min<int64_t>((nv + 255) / 256, 1 << 20);
+  k_w_bins<<<nb, 256, 0, ctx->stream>>>(w, nv, stride, wstep, bin);
   CROC_HIP(hipGetLastError());
   return CROC_OK;
 }

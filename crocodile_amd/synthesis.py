@@ -1022,11 +1022,23 @@ def _src_rows(src, nv):
     return a.reshape(nv, -1) if a.size else None
 
 
+def _w_bins(uv, wstep):
+    """w-plane round-half-even(w / wstep) of every visibility (int64), by the
+    division the gridding kernels make.  torch divides a device tensor by a
+    number as a product with its reciprocal, which puts some w at exact half
+    steps (73.5 at 49) on the neighbouring plane."""
+    w = uv[:, 2]
+    wb = torch.empty(w.shape[0], dtype=torch.int64, device=w.device)
+    _lib.check(_lib.load().croc_w_bins(_lib.ctx(), _lib.ptr(w), w.shape[0], w.stride(0),
+                                       float(wstep), _lib.ptr(wb)))
+    return wb
+
+
 def w_cache_planes(theta, uv, src, wstep, fn, kwargs):
     """Kernel bank with one plane per distinct (w-bin, src row) key and the
     plane-selection arguments for the gridder.  w-bin = round-half-even of
     w / wstep (numpy.round in synthesis.py:793)."""
-    wb = torch.round(uv[:, 2] / wstep).to(torch.int64)
+    wb = _w_bins(uv, wstep)
     src_rows = _src_rows(src, uv.shape[0])
     if src_rows is None or src_rows.shape[1] == 0:
         lo, hi = int(wb.min()), int(wb.max())
@@ -1361,7 +1373,7 @@ def _w_planes(uv, wstep):
     """Per visibility its w-plane round-half-even(w / wstep) (numpy.around,
     wstacking.ipynb cell 10) as int64, and per non-empty plane in ascending
     order: (plane numbers on the host, counts and mean w on the device)."""
-    pl = torch.round(uv[:, 2] / float(wstep)).to(torch.int64)
+    pl = _w_bins(uv, wstep)
     lo, hi = (int(x) for x in torch.stack([pl.min(), pl.max()]).cpu())
     counts = torch.empty(hi - lo + 1, dtype=torch.int64, device=uv.device)
     sums = torch.empty(hi - lo + 1, dtype=torch.float64, device=uv.device)

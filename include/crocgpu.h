@@ -226,6 +226,10 @@ int croc_wstack_grid(croc_ctx *ctx, void *stack, int P, int N, const double *uvw
                      int64_t nv, int64_t stride, double lam, double wstep,
                      int64_t plane0, int ntab, const int32_t *slot_of, const void *vis,
                      int centred);
+/* croc_w_bins: bin[i] (int64) = round-half-even(w[i stride] / wstep), the
+ * w-plane numbers of croc_wplane_sums, croc_wstack_grid and CROC_PLANE_WBIN. */
+int croc_w_bins(croc_ctx *ctx, const double *w, int64_t nv, int64_t stride, double wstep,
+                int64_t *bin);
 /* croc_wplane_sums counts the visibilities of every w-plane t =
  * round-half-even(w / wstep) - plane0, 0 <= t < ntab, and sums their w:
  * count int64 [ntab], sum double [ntab] (overwritten; the planes' mean w of
