@@ -533,7 +533,7 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
                                int32_t *cub, int32_t *cvb) {
   int rc = ctx_enter(ctx);
   if (rc) return rc;
-  CROC_REQUIRE(nv >= 1 && nv < (int64_t)INT32_MAX && stride >= 3 && theta > 0 && wstep > 0 &&
+  CROC_REQUIRE(nv >= 1 && nv < (int64_t)INT32_MAX && stride >= 3 && theta > 0 && wstep != 0 &&
                    chunk >= 1 && nant >= 1,
                CROC_EINVAL, "bad arguments");
   CROC_REQUIRE(uvw && src && order && vstart && gid && rel && gwp && ga1 && ga2 && ngroups &&

@@ -437,7 +437,8 @@ extern "C" int croc_wplane_sums(croc_ctx *ctx, const double *uvw, int64_t nv, in
                                 double *sum) {
   int rc = ctx_enter(ctx);
   if (rc) return rc;
-  CROC_REQUIRE(nv >= 0 && stride >= 3 && wstep > 0 && ntab >= 1, CROC_EINVAL, "bad arguments");
+  CROC_REQUIRE(nv >= 0 && stride >= 3 && wstep != 0 && ntab >= 1, CROC_EINVAL,
+               "bad arguments");
   CROC_REQUIRE(count && sum && (nv == 0 || uvw), CROC_EINVAL, "null array");
   if ((rc = zero_u32_async(ctx, (uint32_t *)count, 2 * (int64_t)ntab))) return rc;
   if ((rc = zero_u32_async(ctx, (uint32_t *)sum, 2 * (int64_t)ntab))) return rc;

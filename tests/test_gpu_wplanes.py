@@ -9,9 +9,11 @@ import torch
 import crocodile_amd.synthesis as G
 from crocodile_amd import _lib
 from crocodile_amd.autograd import WProjectionOperator
+from oracle import awtowers_ref as AWT
 from oracle import synthesis_ref as R
 from oracle import wstacking_ref as WS
 from test_gpu_core import assert_close
+from test_oracle_awtowers import scenario
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +63,24 @@ def test_w_stacking(gpu, wstep, wmax, spread):
     assert numpy.abs(got - ref).max() < 2e-6 * numpy.abs(ref).max()
     ref = WS.w_stacking_imaging(theta, N / theta, uvw, None, vis, wstep)
     got = G.w_stacking_imaging(theta, N / theta, uvw, None, vis, wstep)
+    assert numpy.abs(got - ref).max() < 2e-6 * numpy.abs(ref).max()
+
+
+def test_negative_step(gpu):
+    """w-planes counted downwards: the sub-grid w-stacking form and AW-towers
+    take a negative wstep, as their notebooks' arithmetic does."""
+    print('case negative wstep', flush=True)
+    N, theta, npk = 256, 0.5, 8
+    uvw, vis = case(9, 49.0, 200.0)
+    ref = WS.w_stacking_subgrid_imaging(theta, N / theta, uvw, None, vis, -25.0, npk)
+    got = G.w_stacking_subgrid_imaging(theta, N / theta, uvw, None, vis, -25.0, npk)
+    assert numpy.abs(got - ref).max() < 2e-6 * numpy.abs(ref).max()
+    sc = scenario(seed=3)
+    wk = R.w_kernel_function(sc['l'], sc['m'], -2.0)
+    args = (sc['theta'], sc['lam'], sc['uvw'], sc['src'], sc['vis'], -2.0, sc['S'],
+            sc['margin'], sc['aa_gcf'], sc['aa_sub'], sc['aa_sub2'], sc['aimage'], wk)
+    ref = AWT.aw_towers_imaging(*args)
+    got = G.aw_towers_imaging(*args)
     assert numpy.abs(got - ref).max() < 2e-6 * numpy.abs(ref).max()
 
 
