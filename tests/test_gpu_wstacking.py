@@ -176,3 +176,27 @@ def test_power_of_two_transforms(gpu, N, P):
                                              theta, _lib.ptr(midw)))
     err = (img - ref).abs().pow(2).mean().sqrt()
     assert float(err / (ref - base).abs().pow(2).mean().sqrt()) < 8 * numpy.log2(N) * 2.0 ** -24
+
+
+@pytest.mark.parametrize('N,P', [(256, 5), (512, 3), (1024, 2), (2048, 3)])
+def test_power_of_two_phases(gpu, N, P):
+    """The Fresnel weights of croc_wstack_image are those of croc_wstack_add: a
+    plane holding one cell, the first, transforms to a constant exactly, so the
+    images differ by FP64 roundings of the products and sums alone (at most
+    eight per plane)."""
+    from crocodile_amd import _lib
+    rng = numpy.random.default_rng(N)
+    v = torch.as_tensor(rng.standard_normal(P) + 1j * rng.standard_normal(P),
+                        device='cuda').to(torch.complex64)
+    midw = torch.as_tensor(rng.uniform(-900, 900, P), device='cuda')
+    cells = torch.zeros((P, N, N), dtype=torch.complex64, device='cuda')
+    cells[:, 0, 0] = v
+    flat = v[:, None, None].expand(P, N, N).contiguous()
+    a, b = (torch.zeros((N, N), dtype=torch.complex128, device='cuda') for _ in range(2))
+    L = _lib.load()
+    _lib.check(L.croc_wstack_image(_lib.ctx(), _lib.ptr(a), _lib.ptr(cells), P, N, 0.4,
+                                   _lib.ptr(midw)))
+    _lib.check(L.croc_wstack_add(_lib.ctx(), _lib.ptr(b), _lib.ptr(flat), P, N, 0.4,
+                                 _lib.ptr(midw), 1))
+    bound = 8 * (P + 1) * 2.0 ** -53 * float(v.abs().sum())
+    assert float((a - b).abs().max()) <= bound
