@@ -210,10 +210,11 @@ __global__ void k_awt_keys(const int4 *__restrict__ bin, const int64_t *__restri
   idx[i] = (int32_t)i;
 }
 
-// Per group its plane and antennas, per run its chunk key; vstart's end.
+// Per group its plane and antennas, and for the host its chunk key and start;
+// vstart's end.
 __global__ void k_awt_groups(const uint64_t *__restrict__ gkey, int ng, int64_t nv, AwtRange r,
                              int32_t *__restrict__ gwp, int32_t *__restrict__ ga1,
-                             int32_t *__restrict__ ga2, uint64_t *__restrict__ gcid,
+                             int32_t *__restrict__ ga2, ulonglong2 *__restrict__ gout,
                              int32_t *__restrict__ vstart) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g == 0) vstart[ng] = (int32_t)nv;
@@ -224,7 +225,7 @@ __global__ void k_awt_groups(const uint64_t *__restrict__ gkey, int ng, int64_t 
   ga1[g] = (int32_t)(k % r.nant);
   k /= r.nant;
   gwp[g] = (int32_t)(k % r.P) + r.wp;
-  gcid[g] = k / r.P;
+  gout[g] = make_ulonglong2(k / r.P, (unsigned long long)vstart[g]);
 }
 
 // Sorted visibility v: its group (the last start <= v) and its coordinates
@@ -274,11 +275,14 @@ __global__ void k_awt_locate(const double *__restrict__ rel, int64_t nv, double 
 // transform of a group's pre-grid (times M^2) is
 //   sum over its visibilities of v Y[y] X[x],
 //   X[x] = sum_j gcf[xf][j] W^((xs + j - S)(x - S/2)),  W = exp(2 pi i / M),
-// Y likewise with the rows.  segs[blockIdx.y] = (chunk, first group, end
-// group, out): the workgroup sums its AWD_T x AWD_T pixel tile (blockIdx.x)
-// over the segment's groups -- per group times the pair's A-screen ratio and
-// wkern^-wp, the plane factor taken once per plane -- and writes
-// bins[chunk] times win (out < 0) or the FP64 sum to part[out].
+// Y likewise with the rows.  segs[blockIdx.y] = (first group, first
+// visibility, end visibility, out): the workgroup sums its AWD_T x AWD_T
+// pixel tile (blockIdx.x) over the segment's visibilities -- per group times
+// the pair's A-screen ratio and wkern^-wp, the plane factor taken once per
+// plane -- and writes bins[~out] times win (out < 0) or the FP64 sum to
+// part[out].  A group may be cut between segments: its parts are summed in
+// FP64, like everything above a run of at most AWD_FOLD + AWD_VB - 1
+// visibilities.
 //
 // Work: 8 S^2 operations per visibility and ~30 S^2 per group in registers,
 // no traffic but the screens (L2) and 24 + 32 bytes per visibility.  A
@@ -304,6 +308,7 @@ __device__ __forceinline__ float chunk_window(const float *__restrict__ win, int
 constexpr int AWD_T = 32;    // tile edge (pixels)
 constexpr int AWD_NT = 256;  // threads: column tid % 32, rows 4 (tid / 32) + q
 constexpr int AWD_VB = 16;   // visibilities whose vectors are staged at a time
+constexpr int AWD_FOLD = 32;  // visibilities after which a group's FP32 sum is folded
 constexpr int AWD_MAX_M = 4096;  // twiddle table in LDS: 8 M bytes
 
 __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
   double ax[4] = {0.0, 0.0, 0.0, 0.0}, ay[4] = {0.0, 0.0, 0.0, 0.0};  // finished planes
   double sx[4] = {0.0, 0.0, 0.0, 0.0}, sy[4] = {0.0, 0.0, 0.0, 0.0};  // the open plane
   float ix[4] = {0.f, 0.f, 0.f, 0.f}, iy[4] = {0.f, 0.f, 0.f, 0.f};   // the open group
-  int g = seg.y;
+  int g = seg.x;
   int wp = gwp[g];
   int gend = vstart[g + 1];
   float2 p[4], r[4];  // the open group's screens
@@ -382,9 +387,14 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
     }
   };
   screens();
-  const int v1 = vstart[seg.z];
-  for (int v0 = vstart[g]; v0 < v1; v0 += AWD_VB) {
+  const int v1 = seg.z;
+  int open = seg.y;  // first visibility of the open FP32 sum
+  for (int v0 = seg.y; v0 < v1; v0 += AWD_VB) {
     const int m = min(AWD_VB, v1 - v0);
+    if (v0 - open >= AWD_FOLD) {
+      close_group();
+      open = v0;
+    }
     __syncthreads();  // table written; the previous vectors read
     for (int e = tid; e < m * 2 * AWD_T; e += AWD_NT) {
       const int k = e / (2 * AWD_T), j = e % (2 * AWD_T);
@@ -410,6 +420,7 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
     for (int k = 0; k < m; k++) {
       if (v0 + k == gend) {  // groups hold at least one visibility
         close_group();
+        open = v0 + k;
         g++;
         const int w = gwp[g];
         if (w != wp) close_plane();
@@ -436,7 +447,7 @@ __global__ __launch_bounds__(AWD_NT) void k_awt_direct(
     if (!in[q]) continue;
     if (seg.w < 0) {
       const float w = chunk_window(win, pix[q], S);
-      bins[(int64_t)seg.x * SS + pix[q]] = make_float2((float)ax[q] * w, (float)ay[q] * w);
+      bins[(int64_t)~seg.w * SS + pix[q]] = make_float2((float)ax[q] * w, (float)ay[q] * w);
     } else {
       part[(int64_t)seg.w * SS + pix[q]] = make_double2(ax[q], ay[q]);
     }
@@ -529,15 +540,15 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
                                double theta, double wstep, int chunk, const int64_t *src,
                                int64_t nant, int32_t *order, int32_t *vstart, int32_t *gid,
                                double *rel, int32_t *gwp, int32_t *ga1, int32_t *ga2,
-                               int64_t *ngroups, int64_t *nchunks, int64_t *cstart,
-                               int32_t *cub, int32_t *cvb) {
+                               int64_t *ngroups, int64_t *nchunks, int32_t *vstart_h,
+                               int64_t *cstart, int32_t *cub, int32_t *cvb) {
   int rc = ctx_enter(ctx);
   if (rc) return rc;
   CROC_REQUIRE(nv >= 1 && nv < (int64_t)INT32_MAX && stride >= 3 && theta > 0 && wstep != 0 &&
                    chunk >= 1 && nant >= 1,
                CROC_EINVAL, "bad arguments");
   CROC_REQUIRE(uvw && src && order && vstart && gid && rel && gwp && ga1 && ga2 && ngroups &&
-                   nchunks && cstart && cub && cvb,
+                   nchunks && vstart_h && cstart && cub && cvb,
                CROC_EINVAL, "null array");
   const size_t n = (size_t)nv;
   hipStream_t s = ctx->stream;
@@ -552,7 +563,7 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
   const size_t tb = std::max(t_sort, std::max(t_rle, t_scan));
   char *w = (char *)ws_get(ctx, WS_SORT, 512 + n * (16 + 3 * 8 + 2 * 4) + tb + 256);
   int *small = (int *)ws_get(ctx, WS_SMALL, 256);
-  uint64_t *h = (uint64_t *)host_stage(ctx, sizeof(uint64_t) * n + 256);
+  ulonglong2 *h = (ulonglong2 *)host_stage(ctx, sizeof(ulonglong2) * n + 256);
   if (!w || !small || !h) return CROC_ENOMEM;
   int4 *bin = (int4 *)w;
   key = (uint64_t *)(bin + n);
@@ -596,22 +607,24 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
   const int ng = *(const int *)h;
   t = tb;
   CROC_HIP(hipcub::DeviceScan::ExclusiveSum(temp, t, count, vstart, ng, s));
-  uint64_t *gcid = key;  // the unsorted keys are no longer needed
-  k_awt_groups<<<(unsigned)((ng + 255) / 256), 256, 0, s>>>(gkey, ng, nv, r, gwp, ga1, ga2, gcid,
+  ulonglong2 *gout = (ulonglong2 *)key;  // over key and skey, no longer needed
+  k_awt_groups<<<(unsigned)((ng + 255) / 256), 256, 0, s>>>(gkey, ng, nv, r, gwp, ga1, ga2, gout,
                                                             vstart);
   k_awt_rel<<<nb, 256, 0, s>>>(uvw, nv, stride, order, bin, vstart, ng, theta, wstep, chunk, gid,
                                rel);
   CROC_HIP(hipGetLastError());
-  CROC_HIP(hipMemcpyAsync(h, gcid, sizeof(uint64_t) * ng, hipMemcpyDeviceToHost, s));
+  CROC_HIP(hipMemcpyAsync(h, gout, sizeof(ulonglong2) * ng, hipMemcpyDeviceToHost, s));
   CROC_HIP(hipStreamSynchronize(s));
   int64_t nc = 0;
   for (int g = 0; g < ng; g++) {
-    if (g == 0 || h[g] != h[g - 1]) {
-      cub[nc] = (int32_t)(h[g] / (uint64_t)r.nvb) + r.ub;
-      cvb[nc] = (int32_t)(h[g] % (uint64_t)r.nvb) + r.vb;
+    vstart_h[g] = (int32_t)h[g].y;
+    if (g == 0 || h[g].x != h[g - 1].x) {
+      cub[nc] = (int32_t)(h[g].x / (uint64_t)r.nvb) + r.ub;
+      cvb[nc] = (int32_t)(h[g].x % (uint64_t)r.nvb) + r.vb;
       cstart[nc++] = g;
     }
   }
+  vstart_h[ng] = (int32_t)nv;
   cstart[nc] = ng;
   *ngroups = ng;
   *nchunks = nc;
@@ -620,7 +633,8 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
 
 extern "C" int croc_awt_direct(croc_ctx *ctx, void *bins, int nc, int S, const double *rel,
                                int64_t nv, double lam_sub, int Q, int K, const void *gcf,
-                               const void *vis, const int32_t *vstart, const int64_t *cstart,
+                               const void *vis, const int32_t *vstart,
+                               const int32_t *vstart_h, const int64_t *cstart,
                                const int32_t *gwp, const int32_t *ga1, const int32_t *ga2,
                                const void *ascreen, const float *win, const double *turns,
                                const float *lmag, int64_t max_bytes) {
@@ -631,41 +645,49 @@ extern "C" int croc_awt_direct(croc_ctx *ctx, void *bins, int nc, int S, const d
                    lam_sub > 0 && nc >= 0 && nv >= 0 && nv < (int64_t)INT32_MAX,
                CROC_EINVAL, "bad arguments");
   if (nc == 0 || nv == 0) return CROC_OK;
-  CROC_REQUIRE(bins && rel && gcf && vis && vstart && cstart && gwp && ga1 && ga2 && ascreen &&
+  CROC_REQUIRE(bins && rel && gcf && vis && vstart && vstart_h && cstart && gwp && ga1 && ga2 && ascreen &&
                    win && turns && lmag,
                CROC_EINVAL, "null array");
-  // Segments of at most `seg` groups of one chunk, so that the crowded chunks
-  // at the centre of the uv plane spread over the chip; a chunk of one
-  // segment writes its image itself, the others leave FP64 partial sums
-  // (longer segments where those would exceed max_bytes).
-  const int SS = S * S;
-  int64_t seg = 64, most = 0;
   for (int c = 0; c < nc; c++) {
-    const int64_t n = cstart[c + 1] - cstart[c];
-    CROC_REQUIRE(cstart[c] >= 0 && n > 0 && cstart[c + 1] <= nv, CROC_EINVAL,
-                 "chunk %d holds no groups", c);
-    most = std::max(most, n);
+    const int64_t a = cstart[c], b = cstart[c + 1];
+    CROC_REQUIRE(a >= 0 && a < b && b <= nv, CROC_EINVAL, "chunk %d holds no groups", c);
+    CROC_REQUIRE(vstart_h[a] >= 0 && vstart_h[b] <= nv, CROC_EINVAL, "bad group range");
   }
-  auto parts_at = [&](int64_t len) {
-    int64_t k = 0;
-    for (int c = 0; c < nc; c++) {
-      const int64_t n = (cstart[c + 1] - cstart[c] + len - 1) / len;
-      k += n > 1 ? n : 0;
-    }
-    return k;
-  };
-  while (seg < most && parts_at(seg) * SS * (int64_t)sizeof(double2) > max_bytes) seg *= 2;
+  // Segments of one chunk of at most `groups` groups and `visibs`
+  // visibilities, cutting through groups, so that the crowded chunks at the
+  // centre of the uv plane and the groups of a dense core spread over the
+  // chip; a chunk of one segment writes its image itself, the others leave
+  // FP64 partial sums (longer segments where those would exceed max_bytes).
+  // 512 visibilities, a few times what 64 groups of the sparse arrays hold,
+  // take their workgroups about 0.1 ms.
+  const int SS = S * S;
+  int64_t groups = 64, visibs = 512;
   std::vector<int4> segs, red;
-  int npart = 0;
-  for (int c = 0; c < nc; c++) {
-    const int64_t a = cstart[c], b = cstart[c + 1], n = (b - a + seg - 1) / seg;
-    for (int64_t k = 0; k < n; k++)
-      segs.push_back(make_int4(c, (int)(a + k * seg), (int)std::min(b, a + (k + 1) * seg),
-                               n == 1 ? -1 : npart + (int)k));
-    if (n > 1) {
-      red.push_back(make_int4(c, npart, npart + (int)n, 0));
-      npart += (int)n;
+  int64_t npart;
+  for (;; groups *= 2, visibs *= 2) {
+    segs.clear();
+    red.clear();
+    npart = 0;
+    for (int c = 0; c < nc; c++) {
+      const size_t first = segs.size();
+      int64_t g = cstart[c], v = vstart_h[g];
+      const int64_t gend = cstart[c + 1], vend = vstart_h[gend];
+      while (v < vend) {
+        const int64_t e =
+            std::min<int64_t>(v + visibs, vstart_h[std::min(gend, g + groups)]);
+        CROC_REQUIRE(e > v, CROC_EINVAL, "empty group %lld", (long long)g);
+        segs.push_back(make_int4((int)g, (int)v, (int)e, ~c));
+        v = e;  // in the last group that starts at or before it
+        g = std::upper_bound(vstart_h + g, vstart_h + gend, (int32_t)v) - vstart_h - 1;
+      }
+      const int64_t n = (int64_t)(segs.size() - first);
+      if (n > 1) {
+        red.push_back(make_int4(c, (int)npart, (int)(npart + n), 0));
+        for (int64_t k = 0; k < n; k++) segs[first + k].w = (int)(npart + k);
+        npart += n;
+      }
     }
+    if (npart == 0 || npart * SS * (int64_t)sizeof(double2) <= max_bytes) break;
   }
   const size_t ns = segs.size(), nr = red.size();
   int4 *d = (int4 *)ws_get(ctx, WS_TOWER, sizeof(int4) * (ns + nr));

@@ -1635,6 +1635,7 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     ints = torch.empty((6, nv + 1), dtype=torch.int32, device=dev)
     order, vstart32, gid, gwp32, ga1, ga2 = ints.unbind(0)
     rel = torch.empty((nv, 3), dtype=torch.float64, device=dev)
+    vstart_h = numpy.empty(nv + 1, dtype=numpy.int32)
     cstart_h = numpy.empty(nv + 1, dtype=numpy.int64)
     cub, cvb = numpy.empty((2, nv), dtype=numpy.int32)
     ng, nc = ctypes.c_int64(), ctypes.c_int64()
@@ -1642,13 +1643,13 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
         _lib.ctx(), _lib.ptr(uv), nv, uv.shape[1], float(theta), float(wstep), S - margin,
         _lib.ptr(st), nant, _lib.ptr(order), _lib.ptr(vstart32), _lib.ptr(gid), _lib.ptr(rel),
         _lib.ptr(gwp32), _lib.ptr(ga1), _lib.ptr(ga2), ctypes.byref(ng), ctypes.byref(nc),
-        cstart_h.ctypes.data_as(ctypes.c_void_p), cub.ctypes.data_as(ctypes.c_void_p),
-        cvb.ctypes.data_as(ctypes.c_void_p))
+        vstart_h.ctypes.data_as(ctypes.c_void_p), cstart_h.ctypes.data_as(ctypes.c_void_p),
+        cub.ctypes.data_as(ctypes.c_void_p), cvb.ctypes.data_as(ctypes.c_void_p))
     if rc == _lib.EPLANE:
         raise IndexError('antenna index outside the A-screens')
     _lib.check(rc)
     G, C = ng.value, nc.value
-    cstart_h = cstart_h[:C + 1]
+    vstart_h, cstart_h = vstart_h[:G + 1], cstart_h[:C + 1]
     _, corner = _awt_chunks(theta, lam, S, margin, cub[:C], cvb[:C])
     if dl != 0 or dm != 0:
         vc = vis_t.index_select(0, order[:nv])
@@ -1669,24 +1670,27 @@ def aw_towers_imaging(theta, lam, uvw, src, vis, wstep, subgrid_size, margin, aa
     wk = _dev(wkern, torch.complex128)
     turns = (torch.angle(wk) / (2 * math.pi)).contiguous()
     lmag = torch.log2(torch.abs(wk)).to(torch.float32).contiguous()
-    # Groups of few visibilities are summed directly (croc_awt_direct): ~15 ns
-    # per visibility, where the pre-grids cost ~1 us per (2S)^2 grid and
-    # 5 ns per visibility.  Measured with the awtowers1800 tracks repeated:
-    # S = 128, 1.8 visibilities per group 1.5 / 7.3 ms (direct / pre-grids),
-    # 32 times as many 7.3 / 9.1, 64 times 13.0 / 11.0; S = 64, 1.7 per group
-    # 1.4 / 2.7, 8 times 2.95 / 3.16, 16 times 4.7 / 3.7.  The line is one
-    # visibility per AWT_DIRECT_CELLS pre-grid cells.
+    # Groups of few visibilities are summed directly (croc_awt_direct): ~6 ns
+    # per visibility at S = 128, where the pre-grids cost ~1 us per (2S)^2 grid
+    # and 5 ns per visibility.  Measured with the awtowers1800 tracks repeated
+    # (direct / pre-grids): S = 128, 1.8 visibilities per group 0.88 / 6.5 ms,
+    # 32 times as many 3.3 / 8.4, 128 times 10.7 / 14.3; S = 64, 1.7 per group
+    # 0.72 / 2.1, 16 times 1.06 / 3.0, 128 times 3.7 / 9.9.  The line, one
+    # visibility per AWT_DIRECT_CELLS pre-grid cells (64 a group at S = 128, 16
+    # at S = 64), lies inside the direct sum's range.  It takes the mean: a core's
+    # long groups are cut into segments like the others (64 pairs of 1e4
+    # visibilities in one chunk and plane among 40608 sparse ones: 5.4 / 23.6).
     if nv * AWT_DIRECT_CELLS <= G * M * M and M <= 4096:
         bins = torch.empty((C, S, S), dtype=torch.complex64, device=dev)
         _lib.check(L.croc_awt_direct(
             _lib.ctx(), _lib.ptr(bins), C, S, _lib.ptr(rel), nv, float(lam_sub), Q, K,
             _lib.ptr(gcf), _lib.ptr(vt), _lib.ptr(vstart32),
-            cstart_h.ctypes.data_as(ctypes.c_void_p), _lib.ptr(gwp32), _lib.ptr(ga1),
-            _lib.ptr(ga2), _lib.ptr(at), _lib.ptr(win), _lib.ptr(turns), _lib.ptr(lmag),
-            min(int(max_stack_bytes), 1 << 30)))
+            vstart_h.ctypes.data_as(ctypes.c_void_p), cstart_h.ctypes.data_as(ctypes.c_void_p),
+            _lib.ptr(gwp32), _lib.ptr(ga1), _lib.ptr(ga2), _lib.ptr(at), _lib.ptr(win),
+            _lib.ptr(turns), _lib.ptr(lmag), min(int(max_stack_bytes), 1 << 30)))
     else:
-        bins = _awt_bins_fft(rel, vt, gid, vstart32[:G + 1].cpu().numpy(), cstart_h, gwp32, ga1,
-                             ga2, S, lam_sub, gcf, at, win, turns, lmag, max_stack_bytes)
+        bins = _awt_bins_fft(rel, vt, gid, vstart_h, cstart_h, gwp32, ga1, ga2, S, lam_sub, gcf,
+                             at, win, turns, lmag, max_stack_bytes)
     fb = torch.fft.fftn(bins, dim=(-2, -1))
     corner_t = torch.as_tensor(corner.astype(numpy.int32), device=dev).contiguous()
     for c0 in range(0, C, 65535):

@@ -257,8 +257,9 @@ int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
  * (int64 [nv][2], indices outside [0, nant) are CROC_EPLANE).  Device outputs:
  * order [nv] (sorted -> input index, stable), vstart [nv + 1] (first
  * visibility of each group, and the end), gid and rel [nv] (sorted order), gwp /
- * ga1 / ga2 [nv] (per group).  Host outputs: the group and chunk counts, cstart
- * [nv + 1] (first group of each chunk, and the end), cub / cvb [nv].
+ * ga1 / ga2 [nv] (per group).  Host outputs: the group and chunk counts,
+ * vstart_h [nv + 1] (vstart again), cstart [nv + 1] (first group of each chunk,
+ * and the end), cub / cvb [nv].
  *
  * croc_awt_pregrid grids visibilities [v0, v1) onto stack[gid - g0]
  * ([G][M][M] cf32, M = 2 * subgrid_size) with the separable cf32 table gcf
@@ -278,7 +279,8 @@ int croc_wstack_add(croc_ctx *ctx, void *image, const void *stack, int P, int N,
  * overwritten) = win times the sum over the chunk's groups g in [cstart[c],
  * cstart[c + 1]) (cstart: host [nc + 1]) of S x S cut-out pixels of M^2
  * times the inverse transform of the group's pre-grid (visibilities
- * [vstart[g], vstart[g + 1]), vstart device [ngroups + 1]), each times the
+ * [vstart[g], vstart[g + 1]), vstart [ngroups + 1] on the device and as
+ * vstart_h on the host), each times the
  * screen ratio and wkern^-gwp[g].  No empty groups or chunks; S <= 2048;
  * at most max_bytes of partial sums.
  * Same errors as the check_only croc_awt_pregrid, nothing written on them.
@@ -289,8 +291,8 @@ int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int64_t stride
                     double theta, double wstep, int chunk, const int64_t *src,
                     int64_t nant, int32_t *order, int32_t *vstart, int32_t *gid,
                     double *rel, int32_t *gwp, int32_t *ga1, int32_t *ga2,
-                    int64_t *ngroups, int64_t *nchunks, int64_t *cstart, int32_t *cub,
-                    int32_t *cvb);
+                    int64_t *ngroups, int64_t *nchunks, int32_t *vstart_h,
+                    int64_t *cstart, int32_t *cub, int32_t *cvb);
 int croc_awt_pregrid(croc_ctx *ctx, void *stack, int M, const double *rel, int64_t v0,
                      int64_t v1, double lam_sub, int Q, int K, const void *gcf,
                      const void *vis, const int32_t *gid, int32_t g0, int check_only);
@@ -300,8 +302,8 @@ int croc_awt_apply(croc_ctx *ctx, void *bins, int c0, int nc, const void *stack,
                    const double *turns, const float *lmag);
 int croc_awt_direct(croc_ctx *ctx, void *bins, int nc, int S, const double *rel,
                     int64_t nv, double lam_sub, int Q, int K, const void *gcf,
-                    const void *vis, const int32_t *vstart, const int64_t *cstart,
-                    const int32_t *gwp, const int32_t *ga1, const int32_t *ga2,
+                    const void *vis, const int32_t *vstart, const int32_t *vstart_h,
+                    const int64_t *cstart, const int32_t *gwp, const int32_t *ga1, const int32_t *ga2,
                     const void *ascreen, const float *win, const double *turns,
                     const float *lmag, int64_t max_bytes);
 int croc_awt_place(croc_ctx *ctx, void *grid, int N, const void *bins, int nc, int S,

@@ -131,3 +131,32 @@ def test_direct_and_transformed_groups(gpu, monkeypatch, direct, S, margin, K, b
     got = G.aw_towers_imaging(*args, max_stack_bytes=budget)
     ref = AWT.aw_towers_imaging(*args)
     assert rel(got, ref) < TOL, rel(got, ref)
+
+
+@pytest.mark.parametrize('S,margin,run,budget', [(32, 6, 40_000, 4 << 30),  # one tile, many parts
+                                                 (34, 8, 1000, 4 << 30),    # ragged tiles
+                                                 (64, 16, 40_000, 1)])      # no room for parts
+def test_direct_sum_of_a_long_run(gpu, monkeypatch, S, margin, run, budget):
+    """One antenna pair's long dense run among groups of a few visibilities,
+    summed directly: its equal terms make the worst of a plain FP32 sum (1e-4
+    after 4e4), where sums of at most 47 stay within 47 / 2 roundings of 2^-24
+    = 1.4e-6, inside the bound of this file."""
+    monkeypatch.setattr(G, 'AWT_DIRECT_CELLS', 0)
+    print('case awtowers run S=%d n=%d' % (S, run), flush=True)
+    sc = scenario(seed=6, S=S, margin=margin)
+    uvw = numpy.concatenate([sc['uvw'][:40], numpy.repeat(sc['uvw'][40:41], run, 0),
+                             sc['uvw'][40:]])
+    src = numpy.concatenate([sc['src'][:40], numpy.repeat(sc['src'][40:41], run, 0),
+                             sc['src'][40:]])
+    vis = numpy.concatenate([sc['vis'][:40], numpy.full(run, 1.1 + 0.7j), sc['vis'][40:]])
+    vis = vis.astype(numpy.complex64)
+    wk = R.w_kernel_function(sc['l'], sc['m'], 2.0)
+    args = (sc['theta'], sc['lam'], uvw, src, vis, 2.0, S, margin, sc['aa_gcf'], sc['aa_sub'],
+            sc['aa_sub2'], sc['aimage'], wk)
+    got = G.aw_towers_imaging(*args, max_stack_bytes=budget)
+    # the oracle on one visibility standing for the run
+    one = numpy.concatenate([vis[:40], [numpy.complex128(vis[40]) * run], vis[40 + run:]])
+    keep = numpy.r_[0:41, 40 + run:len(uvw)]
+    ref = AWT.aw_towers_imaging(sc['theta'], sc['lam'], uvw[keep], src[keep],
+                                one.astype(complex), *args[5:])
+    assert rel(got, ref) < TOL, rel(got, ref)
