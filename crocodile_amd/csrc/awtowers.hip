@@ -192,6 +192,10 @@ __global__ void k_awt_range_init(int *range, uint32_t *status) {
   if (threadIdx.x == 6) *status = 0u;
 }
 
+// Groups whose chunk keys and starts come to the host at a time: 1 MiB of the
+// context's pinned staging, which lives as long as the context.
+constexpr int AWG_STAGE = 65536;
+
 struct AwtRange {
   int ub, vb, wp;      // lowest
   int64_t nvb, P, nant;
@@ -563,7 +567,8 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
   const size_t tb = std::max(t_sort, std::max(t_rle, t_scan));
   char *w = (char *)ws_get(ctx, WS_SORT, 512 + n * (16 + 3 * 8 + 2 * 4) + tb + 256);
   int *small = (int *)ws_get(ctx, WS_SMALL, 256);
-  ulonglong2 *h = (ulonglong2 *)host_stage(ctx, sizeof(ulonglong2) * n + 256);
+  ulonglong2 *h = (ulonglong2 *)host_stage(
+      ctx, std::max<size_t>(sizeof(ulonglong2) * std::min<size_t>(n, AWG_STAGE), 256));
   if (!w || !small || !h) return CROC_ENOMEM;
   int4 *bin = (int4 *)w;
   key = (uint64_t *)(bin + n);
@@ -613,15 +618,21 @@ extern "C" int croc_awt_groups(croc_ctx *ctx, const double *uvw, int64_t nv, int
   k_awt_rel<<<nb, 256, 0, s>>>(uvw, nv, stride, order, bin, vstart, ng, theta, wstep, chunk, gid,
                                rel);
   CROC_HIP(hipGetLastError());
-  CROC_HIP(hipMemcpyAsync(h, gout, sizeof(ulonglong2) * ng, hipMemcpyDeviceToHost, s));
-  CROC_HIP(hipStreamSynchronize(s));
   int64_t nc = 0;
-  for (int g = 0; g < ng; g++) {
-    vstart_h[g] = (int32_t)h[g].y;
-    if (g == 0 || h[g].x != h[g - 1].x) {
-      cub[nc] = (int32_t)(h[g].x / (uint64_t)r.nvb) + r.ub;
-      cvb[nc] = (int32_t)(h[g].x % (uint64_t)r.nvb) + r.vb;
-      cstart[nc++] = g;
+  uint64_t last = 0;
+  for (int g0 = 0; g0 < ng; g0 += AWG_STAGE) {
+    const int m = std::min(AWG_STAGE, ng - g0);
+    CROC_HIP(hipMemcpyAsync(h, gout + g0, sizeof(ulonglong2) * m, hipMemcpyDeviceToHost, s));
+    CROC_HIP(hipStreamSynchronize(s));
+    for (int k = 0; k < m; k++) {
+      const uint64_t cid = h[k].x;
+      vstart_h[g0 + k] = (int32_t)h[k].y;
+      if (g0 + k == 0 || cid != last) {
+        cub[nc] = (int32_t)(cid / (uint64_t)r.nvb) + r.ub;
+        cvb[nc] = (int32_t)(cid % (uint64_t)r.nvb) + r.vb;
+        cstart[nc++] = g0 + k;
+      }
+      last = cid;
     }
   }
   vstart_h[ng] = (int32_t)nv;

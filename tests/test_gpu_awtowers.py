@@ -160,3 +160,51 @@ def test_direct_sum_of_a_long_run(gpu, monkeypatch, S, margin, run, budget):
     ref = AWT.aw_towers_imaging(sc['theta'], sc['lam'], uvw[keep], src[keep],
                                 one.astype(complex), *args[5:])
     assert rel(got, ref) < TOL, rel(got, ref)
+
+
+@pytest.mark.parametrize('nv,spread', [(1, 1), (65_536, 65_536), (65_537, 65_537),
+                                       (140_000, 131_073), (300_000, 900)])
+def test_groups(gpu, nv, spread):
+    """croc_awt_groups against NumPy: group and chunk tables that come to the
+    host in one piece and in several, with chunks across the cuts."""
+    import ctypes
+    from crocodile_amd import _lib
+    print('case awt groups nv=%d' % nv, flush=True)
+    rng = numpy.random.default_rng(nv)
+    theta, wstep, chunk, nant = 0.1, 3.0, 20, 700
+    which = rng.permutation(numpy.arange(nv) % spread)   # `spread` groups
+    chunks = which % 11
+    uvw = numpy.stack([(chunks % 4 - 1.3) * chunk / theta, (chunks // 4 + 0.2) * chunk / theta,
+                       (which // 11 % 5) * wstep + rng.uniform(-1, 1, nv)], 1)
+    src = numpy.stack([which // 55 % nant, which // 55 // nant], 1)
+    d = lambda n, t: torch.zeros(n, dtype=t, device=gpu)  # noqa: E731
+    order, vstart, gid, gwp, ga1, ga2 = (d(nv + 1, torch.int32) for _ in range(6))
+    rel = d((nv, 3), torch.float64)
+    vstart_h, cstart = numpy.zeros(nv + 1, numpy.int32), numpy.zeros(nv + 1, numpy.int64)
+    cub, cvb = numpy.zeros((2, nv), numpy.int32)
+    ng, nc = ctypes.c_int64(), ctypes.c_int64()
+    host = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    ud, sd = torch.as_tensor(uvw, device=gpu), torch.as_tensor(src, device=gpu)
+    _lib.check(_lib.load().croc_awt_groups(
+        _lib.ctx(), _lib.ptr(ud), nv, 3, theta, wstep, chunk, _lib.ptr(sd), nant,
+        *(_lib.ptr(t) for t in (order, vstart, gid, rel, gwp, ga1, ga2)), ctypes.byref(ng),
+        ctypes.byref(nc), host(vstart_h), host(cstart), host(cub), host(cvb)))
+    G_, C = ng.value, nc.value
+    ub, vb = (numpy.floor(uvw[:, k] * theta / chunk + 0.5).astype(int) for k in (0, 1))
+    wp = numpy.around(uvw[:, 2] / wstep).astype(int)
+    perm = numpy.lexsort((src[:, 1], src[:, 0], wp, vb, ub))   # stable
+    key = numpy.stack([ub, vb, wp, src[:, 0], src[:, 1]], 1)[perm]
+    new = numpy.r_[True, (key[1:] != key[:-1]).any(1)]
+    starts = numpy.flatnonzero(new)
+    assert G_ == len(starts) == spread
+    eq = numpy.testing.assert_array_equal
+    eq(order[:nv].cpu().numpy(), perm)
+    eq(vstart[:G_ + 1].cpu().numpy(), numpy.r_[starts, nv])
+    eq(vstart_h[:G_ + 1], numpy.r_[starts, nv])
+    eq(gid[:nv].cpu().numpy(), numpy.cumsum(new) - 1)
+    for got, col in ((gwp, 2), (ga1, 3), (ga2, 4)):
+        eq(got[:G_].cpu().numpy(), key[starts, col])
+    cnew = numpy.r_[True, (key[starts][1:, :2] != key[starts][:-1, :2]).any(1)]
+    assert C == cnew.sum()
+    eq(cstart[:C + 1], numpy.r_[numpy.flatnonzero(cnew), G_])
+    eq(numpy.stack([cub[:C], cvb[:C]], 1), key[starts][cnew, :2])
