@@ -227,25 +227,46 @@ int direct_end(croc_ctx *ctx, volatile uint32_t *host) {
 
 }  // namespace
 
-// Taps (visibilities times max_support^2) up to which the direct path is the
-// faster one, measured per call against the tile path (us, direct / tile):
-//   gridding, bound by the 64-bit atomics into the accumulator beyond L2:
-//     N = 256:  S = 8, 2e4 visibilities 91 / 148, 6e4 176 / 154;
-//     N = 2048: S = 15, 5e3 97 / 174, 2e4 193 / 229, 6e4 444 / 254;
-//   degridding, bound by L2 reads of grid and taps:
-//     N = 256:  S = 15, 1.3e5 74 / 158; S = 32, 6e4 95 / 177;
-//     N = 2048: S = 15, 1.3e5 105 / 143; S = 32, 6e4 120 / 168, 1.3e5 211 / 200.
-constexpr int64_t DIRECT_GRID_TAPS = 3 << 20;
-constexpr int64_t DIRECT_DEGRID_TAPS = 64 << 20;
+// Where the direct path is the faster one, measured per call against the tile
+// path (us, direct / tile; one plane unless said otherwise).
+//
+// Gridding is bound by the 64-bit atomics into the accumulator, and by how many
+// of them fall on one cell, which the tile path adds up in LDS: 24 ns per
+// visibility (S = 8) when all share one window.  So the line is not drawn where
+// spread visibilities break even (1e4 to 2e5) but where those of a core do,
+// normal with a sigma of 4 cells; there nv S is about the same at every S from
+// 4 to 32.  N = 256, S = 8, 5120 visibilities: spread 57 / 101, core 124 / 114,
+// one window 169 / 115 (at 49152: 149 / 113, 734 / 110, 1227 / 107); N = 2048,
+// S = 15, 2730: 90 / 229 with 100 planes (at 13981 with one: 157 / 199, core
+// 565 / 151).  Below S = 8 the count is bounded (S = 1, 196608, core: 238 / 137).
+// N = 8192 and 30000 lie on the same side (433 / 596, 5304 / 5449), and so does a
+// bank of 197 MB (115 / 198).
+constexpr int64_t DIRECT_GRID_ROWS = 40960;  // visibilities times max(S, 8)
+//
+// Degridding is bound by the visibilities (0.15 ns each up to S = 8) and then by
+// L2 reads of grid and taps: taps (visibilities times S^2) set the line, twice
+// as far out with kernel banks that crowd an L2 of 4 MiB, which the tile path
+// reads plane group by plane group.
+//   Small banks, N = 2048: S = 15, 149130 128 / 141, 298260 212 / 184; S = 32,
+//     32768 86 / 151, 65536 133 / 163, 1.3e5 211 / 200; S = 8, 524288 154 / 222;
+//     S = 1, 1.7e7 2472 / 3069.  N = 8192 and 30000, S = 8, 524288: 185 / 513 and
+//     228 / 3654.
+//   100 planes, Q = 8, N = 2048: S = 8 (3 MiB), 1048576 291 / 332; S = 15 (11
+//     MiB), 298260 273 / 413; 150 planes, S = 31, 69832: 211 / 554.
+constexpr int64_t DIRECT_DEGRID_TAPS = 32 << 20;
+constexpr int64_t DIRECT_BANK_BYTES = 2 << 20;
 
 bool direct_grid_wins(const BinArgs &a, int max_support) {
   return max_support >= 1 && max_support <= 64 && a.nv > 0 &&
-         a.nv <= DIRECT_GRID_TAPS / ((int64_t)max_support * max_support);
+         a.nv <= DIRECT_GRID_ROWS / std::max(max_support, 8);
 }
 
 bool direct_degrid_wins(const BinArgs &a, int max_support) {
-  return max_support >= 1 && max_support <= 64 && a.nv > 0 &&
-         a.nv <= DIRECT_DEGRID_TAPS / ((int64_t)max_support * max_support);
+  if (max_support < 1 || max_support > 64 || a.nv <= 0) return false;
+  const int64_t row = (int64_t)a.Q * max_support;
+  const double bank = 8.0 * (double)a.nplanes * (a.separable ? (double)row : (double)row * row);
+  const int64_t taps = DIRECT_DEGRID_TAPS * (bank > DIRECT_BANK_BYTES ? 2 : 1);
+  return a.nv <= taps / ((int64_t)max_support * max_support);
 }
 
 int direct_grid(croc_ctx *ctx, const BinArgs &a, void *grid, const void *vis, const void *kern,
