@@ -64,37 +64,33 @@ __global__ __launch_bounds__(BIN_NT) void k_bin_count(
 }
 
 // Item slots: slot t < ntiles is tile t of the tile-major list; slot ntiles
-// + r * ntiles + t is tile t's records of range r (groups [r * ngroups / nr,
-// (r + 1) * ngroups / nr)) in the range-major per-XCD list.  scount[slot] =
-// items the slot needs; the record offsets are copied to the scatter
-// cursors.
-__device__ __forceinline__ uint32_t slot_items(int i, int ntiles, int ngroups, int nr, int chunk,
+// + g * ntiles + t is tile t's records of plane group g in the group-major
+// per-XCD list.  scount[slot] = items the slot needs; the record offsets are
+// copied to the scatter cursors.
+__device__ __forceinline__ uint32_t slot_items(int i, int ntiles, int ngroups, int chunk,
                                                int order, const uint32_t *offset) {
   uint32_t c = 0;
   if (i < ntiles) {
     if (order & ITEMS_BY_TILE) c = offset[(i + 1) * ngroups] - offset[i * ngroups];
   } else if (order & ITEMS_BY_GROUP) {
-    const int q = i - ntiles, r = q / ntiles, t = q - r * ntiles;
-    // one range per group is what bin_visibilities asks for
-    const int ga = nr == ngroups ? r : r * ngroups / nr;
-    const int gb = nr == ngroups ? r + 1 : (r + 1) * ngroups / nr;
-    c = offset[t * ngroups + gb] - offset[t * ngroups + ga];
+    const int q = i - ntiles, g = q / ntiles, t = q - g * ntiles;
+    c = offset[t * ngroups + g + 1] - offset[t * ngroups + g];
   }
   return (c + chunk - 1) / chunk;
 }
 
-__global__ void k_item_counts(int ntiles, int ngroups, int nr, int chunk, int order, int nbins,
+__global__ void k_item_counts(int ntiles, int ngroups, int chunk, int order, int nbins,
                               const uint32_t *__restrict__ offset,
                               uint32_t *__restrict__ cursor, uint32_t *__restrict__ scount) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nbins) cursor[i] = offset[i];
-  const int nslots = ntiles * (1 + nr);
+  const int nslots = ntiles * (1 + ngroups);
   if (i >= nslots) return;
-  scount[i] = slot_items(i, ntiles, ngroups, nr, chunk, order, offset);
+  scount[i] = slot_items(i, ntiles, ngroups, chunk, order, offset);
 }
 
 // Slot s's first record and end record.
-__device__ __forceinline__ void slot_range(int s, int ntiles, int ngroups, int nr,
+__device__ __forceinline__ void slot_range(int s, int ntiles, int ngroups,
                                            const uint32_t *__restrict__ offset, int *t,
                                            uint32_t *s0, uint32_t *s1) {
   if (s < ntiles) {
@@ -102,21 +98,20 @@ __device__ __forceinline__ void slot_range(int s, int ntiles, int ngroups, int n
     *s0 = offset[s * ngroups];
     *s1 = offset[(s + 1) * ngroups];
   } else {
-    const int q = s - ntiles, r = q / ntiles;
-    *t = q - r * ntiles;
-    const int ga = (int)((int64_t)r * ngroups / nr), gb = (int)((int64_t)(r + 1) * ngroups / nr);
-    *s0 = offset[*t * ngroups + ga];
-    *s1 = offset[*t * ngroups + gb];
+    const int q = s - ntiles, g = q / ntiles;
+    *t = q - g * ntiles;
+    *s0 = offset[*t * ngroups + g];
+    *s1 = offset[*t * ngroups + g + 1];
   }
 }
 
 // One thread per item (items of all slots numbered by soff, the tile-major
 // list first): finds its slot by binary search over soff and writes {tile,
-// first, end}, the per-XCD list renumbered from 0.  Threads below nr + 1
-// also write gstart for the first group of each range and the item counts,
-// and the first XCD_QUEUES reset the queue heads.  An error status leaves
-// both lists empty, so that no output is modified.
-__global__ void k_item_write(int ntiles, int ngroups, int nr, int chunk, int max_total,
+// first, end}, the per-XCD list renumbered from 0.  Threads up to ngroups
+// also write gstart for each group and the item counts, and the first
+// XCD_QUEUES reset the queue heads.  An error status leaves both lists empty,
+// so that no output is modified.
+__global__ void k_item_write(int ntiles, int ngroups, int chunk, int max_total,
                              const uint32_t *__restrict__ offset,
                              const uint32_t *__restrict__ scount,
                              const uint32_t *__restrict__ soff, int4 *__restrict__ items,
@@ -125,18 +120,18 @@ __global__ void k_item_write(int ntiles, int ngroups, int nr, int chunk, int max
                              const uint32_t *__restrict__ status,
                              uint32_t *__restrict__ qheads) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nslots = ntiles * (1 + nr);
+  const int nslots = ntiles * (1 + ngroups);
   const bool failed = *status != 0;
   const uint32_t base_g = soff[ntiles];  // items of the tile-major list
   const uint32_t total = soff[nslots - 1] + scount[nslots - 1];
   if (i < XCD_QUEUES) qheads[i] = 0;
-  if (i <= nr) {
-    if (i == nr) {
+  if (i <= ngroups) {
+    if (i == ngroups) {
       *nitems = failed ? 0u : base_g;
       *nitems_g = failed ? 0u : total - base_g;
       gstart[ngroups] = failed ? 0u : total - base_g;
     } else {
-      gstart[(int64_t)i * ngroups / nr] = failed ? 0u : soff[ntiles + i * ntiles] - base_g;
+      gstart[i] = failed ? 0u : soff[ntiles + i * ntiles] - base_g;
     }
   }
   if (failed || i >= max_total || (uint32_t)i >= total) return;
@@ -149,7 +144,7 @@ __global__ void k_item_write(int ntiles, int ngroups, int nr, int chunk, int max
   }
   int t;
   uint32_t s0, s1;
-  slot_range(lo, ntiles, ngroups, nr, offset, &t, &s0, &s1);
+  slot_range(lo, ntiles, ngroups, offset, &t, &s0, &s1);
   const uint32_t k = (uint32_t)i - soff[lo];
   const uint32_t a = s0 + k * (uint32_t)chunk;
   const int4 item = make_int4(t, (int)a, (int)min(s1, a + (uint32_t)chunk), 0);
@@ -211,7 +206,7 @@ __device__ __forceinline__ uint32_t block_scan(int n, F f, P put) {
 // Measured 5 us at 1000 slots and 39 us at 16000, against 11 + 9 + 5 us and
 // four more launches: the one workgroup up to PLAN_MAX slots.
 constexpr int PLAN_MAX = 8192;
-__global__ __launch_bounds__(BIN_NT) void k_bin_plan(int ntiles, int ngroups, int nr, int chunk,
+__global__ __launch_bounds__(BIN_NT) void k_bin_plan(int ntiles, int ngroups, int chunk,
                                                      int order, int nbins,
                                                      const uint32_t *__restrict__ count,
                                                      uint32_t *offset,
@@ -227,9 +222,9 @@ __global__ __launch_bounds__(BIN_NT) void k_bin_plan(int ntiles, int ngroups, in
   __threadfence_block();
   __syncthreads();  // the offsets are written before other threads read them
   block_scan(
-      ntiles * (1 + nr),
+      ntiles * (1 + ngroups),
       [&](int i) {
-        const uint32_t c = slot_items(i, ntiles, ngroups, nr, chunk, order, offset);
+        const uint32_t c = slot_items(i, ntiles, ngroups, chunk, order, offset);
         scount[i] = c;
         return c;
       },
@@ -348,9 +343,7 @@ int bin_visibilities(croc_ctx *ctx, WsSet &set, const BinArgs &a, int max_suppor
 
   p.loc = (uint4 *)ws_get_in(ctx, set, WS_LOC, sizeof(uint4) * a.nv);
   p.rec = (uint4 *)ws_get_in(ctx, set, WS_REC, sizeof(uint4) * a.nv);
-  // Ranges of the per-XCD list: one per group, at least one per queue.
-  const int nr = p.ngroups;
-  const int nslots = p.ntiles * (1 + nr);
+  const int nslots = p.ntiles * (1 + p.ngroups);
   size_t scan_bytes = 0, t_bytes = 0;
   CROC_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, t_bytes, (const uint32_t *)nullptr,
                                             (uint32_t *)nullptr, p.nbins + 1, ctx->stream));
@@ -399,23 +392,23 @@ int bin_visibilities(croc_ctx *ctx, WsSet &set, const BinArgs &a, int max_suppor
   }
   // record offsets (bins tile-major, offset[nbins] = total), then the items
   if (std::max(p.nbins, nslots) <= PLAN_MAX) {
-    k_bin_plan<<<1, BIN_NT, 0, s>>>(p.ntiles, p.ngroups, nr, p.chunk, order, p.nbins, p.count,
+    k_bin_plan<<<1, BIN_NT, 0, s>>>(p.ntiles, p.ngroups, p.chunk, order, p.nbins, p.count,
                                     p.offset, p.cursor, scount, soff);
   } else {
     t_bytes = scan_bytes;
     CROC_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp, t_bytes, p.count, p.offset,
                                               p.nbins + 1, s));
     const int nth = std::max(p.nbins, nslots);
-    k_item_counts<<<(nth + 255) / 256, 256, 0, s>>>(p.ntiles, p.ngroups, nr, p.chunk, order,
+    k_item_counts<<<(nth + 255) / 256, 256, 0, s>>>(p.ntiles, p.ngroups, p.chunk, order,
                                                     p.nbins, p.offset, p.cursor, scount);
     t_bytes = scan_bytes;
     CROC_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp, t_bytes, scount, soff, nslots, s));
   }
   // at most max_items per list
   const int max_total = (int)std::min<int64_t>(2 * p.max_items, INT32_MAX);
-  const int nthr = std::max(max_total, std::max(nr + 1, XCD_QUEUES));
+  const int nthr = std::max(max_total, std::max(p.ngroups + 1, XCD_QUEUES));
   k_item_write<<<(nthr + 255) / 256, 256, 0, s>>>(
-      p.ntiles, p.ngroups, nr, p.chunk, max_total, p.offset, scount, soff, p.items, p.items_g,
+      p.ntiles, p.ngroups, p.chunk, max_total, p.offset, scount, soff, p.items, p.items_g,
       p.gstart, p.nitems, p.nitems_g, p.status, p.qhead);
   if (nblk > 0) {
     if (spread)
