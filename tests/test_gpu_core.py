@@ -146,6 +146,36 @@ def random_case(rng, N, S, Q, nv, planes=1, separable=False, margin=None):
     return tables, p, v
 
 
+def planned_grid(gcf, a, p, src, v):
+    """convgrid through a plan."""
+    plan = make_plan(gcf, a, p, src)
+    g = torch.zeros(a.shape, dtype=torch.complex64, device='cuda')
+    plan.grid(g, torch.as_tensor(v, device='cuda').to(torch.complex64))
+    a += g.cpu().numpy()
+
+
+def planned_degrid(gcf, a, p, src=None):
+    """convdegrid through a plan."""
+    out = torch.empty(len(p), dtype=torch.complex64, device='cuda')
+    make_plan(gcf, a, p, src).degrid(torch.as_tensor(a, device='cuda').to(torch.complex64), out)
+    return out.cpu().numpy()
+
+
+def make_plan(gcf, a, p, src):
+    tables = [gcf] if src is None else list(gcf)
+    bank = G.KernelBank.from_tables(tables, tables[0].ndim == 2)
+    mode, vp = _lib.PLANE_SINGLE, None
+    if src is not None:
+        mode, vp = _lib.PLANE_INDEX, torch.as_tensor(src[:, 0].astype(numpy.int32), device='cuda')
+    return G.GridPlan(bank, len(a), torch.as_tensor(p, device='cuda'), 1.0, mode, vp)
+
+
+# One-shot calls of few visibilities take the direct kernels, which know no
+# tiles, chunks or plane groups; a plan always takes the tile kernels.
+PATHS = {'one-shot': (G.convgrid, G.convdegrid), 'plan': (planned_grid, planned_degrid)}
+both_paths = pytest.mark.parametrize('path', sorted(PATHS))
+
+
 CASES = [
     # N, S, Q, nv, planes, separable
     (64, 4, 2, 3000, 1, False),
@@ -159,8 +189,10 @@ CASES = [
 ]
 
 
+@both_paths
 @pytest.mark.parametrize('N,S,Q,nv,planes,separable', CASES)
-def test_convgrid_convdegrid_parity(gpu, N, S, Q, nv, planes, separable):
+def test_convgrid_convdegrid_parity(gpu, N, S, Q, nv, planes, separable, path):
+    convgrid, convdegrid = PATHS[path]
     print('case N=%d S=%d Q=%d nv=%d planes=%d sep=%d' % (N, S, Q, nv, planes, separable),
           flush=True)
     rng = numpy.random.default_rng(N * 7 + S)
@@ -172,17 +204,19 @@ def test_convgrid_convdegrid_parity(gpu, N, S, Q, nv, planes, separable):
     ref = numpy.zeros((N, N), dtype=complex)
     cgrid.convgrid(bank, ref, p, v, vplane.astype(numpy.int32) if planes > 1 else None)
     a = numpy.zeros((N, N), dtype=complex)
-    G.convgrid(gcf, a, p, src, v)
+    convgrid(gcf, a, p, src, v)
     assert_close(a, ref, what='grid')
     vref = cgrid.convdegrid(bank, ref, p, vplane.astype(numpy.int32) if planes > 1 else None)
-    vd = G.convdegrid(gcf, ref, p, src)
+    vd = convdegrid(gcf, ref, p, src)
     assert_close(vd, vref, what='degrid')
 
 
-def test_every_support_size(gpu):
+@both_paths
+def test_every_support_size(gpu, path):
     """Supports 1..64: the window walk splits S*S taps into unmasked blocks
     of 1024 / 512 / 256 taps and one masked remainder, and finds each tap's
-    row with a 24-bit reciprocal multiply; every split and every S is hit."""
+    row with a 24-bit reciprocal multiply; every split and every S is hit, in the direct and the tile kernels."""
+    convgrid, convdegrid = PATHS[path]
     for S in range(1, 65):
         for separable in (False, True):
             rng = numpy.random.default_rng(1000 + 2 * S + separable)
@@ -192,9 +226,9 @@ def test_every_support_size(gpu):
             ref = numpy.zeros((N, N), dtype=complex)
             cgrid.convgrid(bank, ref, p, v, None)
             a = numpy.zeros((N, N), dtype=complex)
-            G.convgrid(tables[0], a, p, None, v)
+            convgrid(tables[0], a, p, None, v)
             assert_close(a, ref, what='grid S=%d sep=%d' % (S, separable))
-            vd = G.convdegrid(tables[0], ref, p, None)
+            vd = convdegrid(tables[0], ref, p, None)
             assert_close(vd, cgrid.convdegrid(bank, ref, p, None),
                          what='degrid S=%d sep=%d' % (S, separable))
 
@@ -332,7 +366,9 @@ def test_make_grid_hermitian(gpu):
         assert_close(t.cpu().numpy(), ref, what='hermitian c64')
 
 
-def test_tiling_knobs_do_not_change_results(gpu):
+@both_paths
+def test_tiling_knobs_do_not_change_results(gpu, path):
+    convgrid, convdegrid = PATHS[path]
     rng = numpy.random.default_rng(12)
     (gcf,), p, v = random_case(rng, 256, 12, 4, 20000)
     ref = numpy.zeros((256, 256), dtype=complex)
@@ -341,18 +377,20 @@ def test_tiling_knobs_do_not_change_results(gpu):
         for tile, chunk in [(16, 64), (48, 1000), (80, 100000)]:
             _lib.set_tuning(tile, chunk)
             a = numpy.zeros((256, 256), dtype=complex)
-            G.convgrid(gcf, a, p, None, v)
+            convgrid(gcf, a, p, None, v)
             assert_close(a, ref, what='tile=%d chunk=%d' % (tile, chunk))
-            assert_close(G.convdegrid(gcf, ref, p), R.convdegrid(gcf, ref, p),
+            assert_close(convdegrid(gcf, ref, p), R.convdegrid(gcf, ref, p),
                          what='degrid tile=%d' % tile)
     finally:
         _lib.set_tuning()
 
 
-def test_plane_groups_do_not_change_results(gpu):
+@both_paths
+def test_plane_groups_do_not_change_results(gpu, path):
     """Binning by (tile, kernel-bank slice): every group size, from one
     group to a group per fraction of a plane, gives the oracle's degridded
     visibilities and bit-identical grids."""
+    convgrid, convdegrid = PATHS[path]
     rng = numpy.random.default_rng(14)
     N, S, Q, nv, planes = 256, 12, 4, 30000, 12
     tables, p, v = random_case(rng, N, S, Q, nv, planes)
@@ -368,10 +406,10 @@ def test_plane_groups_do_not_change_results(gpu):
         for group_kib in (0, 1, 2, 8, 64, 2048):
             _lib.set_tuning(0, 1024, group_kib)
             a = numpy.zeros((N, N), dtype=complex)
-            G.convgrid(gcf, a, p, src, v)
+            convgrid(gcf, a, p, src, v)
             assert_close(a, ref, what='grid group_kib=%d' % group_kib)
             grids.append(a)
-            assert_close(G.convdegrid(gcf, ref, p, src), vref,
+            assert_close(convdegrid(gcf, ref, p, src), vref,
                          what='degrid group_kib=%d' % group_kib)
     finally:
         _lib.set_tuning()

@@ -60,7 +60,8 @@ def test_tile_path_nonfinite_visibilities(gpu, separable):
 
 def test_tile_path_nonfinite_tap(gpu):
     """A NaN tap in one (yf, xf) table: the cells of exactly the visibilities
-    using that table, at that tap."""
+    using that table, at that tap; one-shot (the direct kernels at this size) and
+    planned (the tile kernels)."""
     rng = numpy.random.default_rng(12)
     N, S, Q, nv = 128, 6, 4, 4000
     kern = rng.standard_normal((Q, Q, S, S)) + 1j * rng.standard_normal((Q, Q, S, S)) + 0.1
@@ -72,6 +73,11 @@ def test_tile_path_nonfinite_tap(gpu):
     got = numpy.zeros((N, N), complex)
     G.convgrid(kern, got, p, None, v)
     compare(got, ref)
+    plan = G.GridPlan(G.KernelBank.from_tables([kern], separable=False), N,
+                      torch.as_tensor(p, device=gpu), 1.0)
+    g = torch.zeros((N, N), dtype=torch.complex64, device=gpu)
+    plan.grid(g, torch.as_tensor(v, device=gpu).to(torch.complex64))
+    compare(g.cpu().numpy().astype(complex), ref)
 
 
 @pytest.mark.parametrize('kind', ['nearest', 'separable'])
