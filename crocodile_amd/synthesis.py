@@ -1385,6 +1385,18 @@ def _w_planes(uv, wstep):
     return pl, lo, hi - lo + 1, (nz + lo).cpu().tolist(), counts[nz], midw
 
 
+# croc_wstack_image (transforms with the plane sum fused) is written for N = 256,
+# 512, 1024 and 2048: whole rows and at least four columns of a power of two in a
+# workgroup's LDS.  It reads and writes the stack less often, which pays once
+# the stack leaves the last-level cache; there the library transform and
+# croc_wstack_add take (fused / library, us): N = 256, 130 planes 152 / 118, 260
+# 189 / 221; N = 512, 32 planes 153 / 145, 48 172 / 209, 260 440 / 1078; N = 1024,
+# 8 planes 165 / 150, 16 217 / 276, 65 525 / 1151; N = 2048, one plane 89 / 112, 65
+# 2166 / 4549.  Other N (other radices; 4096, whose tile would be two columns
+# wide) have the library alone: N = 2000, 65 planes 4588, N = 4096 21091.
+WSTACK_FUSED_CELLS = 10_000_000
+
+
 def w_stacking_imaging(theta, lam, uvw, src, vis, wstep, max_stack_bytes=4 << 30):
     """Full-grid w-stacking (wstacking.ipynb cell 10, JSON lines 191-240):
     the visibilities of each w-plane round(w / wstep) are imaged nearest-cell
@@ -1424,8 +1436,7 @@ def w_stacking_imaging(theta, lam, uvw, src, vis, wstep, max_stack_bytes=4 << 30
                                       uv.shape[0], uv.shape[1], float(lam), float(wstep),
                                       lo, ntab, _lib.ptr(slot_of), _lib.ptr(vt), centred))
         mw = midw[b0:b0 + P].contiguous()
-        if N in (256, 512, 1024, 2048):
-            # power-of-two grids: transforms with the plane sum fused
+        if N in (256, 512, 1024, 2048) and (N == 2048 or P * N * N >= WSTACK_FUSED_CELLS):
             _lib.check(L.croc_wstack_image(_lib.ctx(), _lib.ptr(image), _lib.ptr(st), P, N,
                                            float(theta), _lib.ptr(mw)))
             continue

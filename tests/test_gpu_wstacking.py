@@ -35,14 +35,16 @@ def rel(got, ref):
     return numpy.abs(got - ref).max() / numpy.abs(ref).max()
 
 
-@pytest.mark.parametrize('N,theta,wstep,budget', [(256, 0.5, 10.0, 4 << 30),
-                                                   (256, 0.5, 10.0, 5 * 256 * 256 * 8),
-                                                   (255, 0.5, 10.0, 4 << 30),
-                                                   (130, 0.25, 7.0, 3 * 130 * 130 * 8)])
-def test_full_grid_matches_oracle(gpu, N, theta, wstep, budget):
+@pytest.mark.parametrize('N,theta,wstep,budget,fused', [
+    (256, 0.5, 10.0, 4 << 30, True), (256, 0.5, 10.0, 4 << 30, False),
+    (256, 0.5, 10.0, 5 * 256 * 256 * 8, True), (256, 0.5, 10.0, 5 * 256 * 256 * 8, False),
+    (255, 0.5, 10.0, 4 << 30, False), (130, 0.25, 7.0, 3 * 130 * 130 * 8, False)])
+def test_full_grid_matches_oracle(gpu, monkeypatch, N, theta, wstep, budget, fused):
     """Even N (centring folded into the kernels), odd N (shifted FFTs), and
-    stacks split into batches of 5 and 3 planes."""
-    print('case wstack full N=%d budget=%d' % (N, budget), flush=True)
+    stacks split into batches of 5 and 3 planes; the fused transforms and the
+    library's."""
+    print('case wstack full N=%d budget=%d fused=%s' % (N, budget, fused), flush=True)
+    monkeypatch.setattr(G, 'WSTACK_FUSED_CELLS', 0 if fused else 1 << 60)
     lam, uvw, vis = case(N, N, theta, 6000, 0.45 * N / theta * 0.5, wstep)
     ref = WS.w_stacking_imaging(theta, lam, uvw, None, vis, wstep)
     got = G.w_stacking_imaging(theta, lam, uvw, None, vis, wstep, max_stack_bytes=budget)
