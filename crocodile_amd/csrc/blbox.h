@@ -8,8 +8,8 @@ constexpr int BL_BOX = 600;  // cells per wavefront: 19 KiB a workgroup
 constexpr int bl_box_pitch(int bw) { return bw | 1; }
 
 // Whether windows spanning bw x bh cells fit the box.  Each extent can be the
-// whole grid's (65536), whose product no int holds: the factors are bounded
-// first.
+// whole grid's (65536), whose product no int holds: rows past the box's cells
+// count as one more than these.
 constexpr bool bl_box_fits(int bw, int bh) {
-  return bh <= BL_BOX && bl_box_pitch(bw) <= BL_BOX && bh * bl_box_pitch(bw) <= BL_BOX;
+  return (bh < BL_BOX + 1 ? bh : BL_BOX + 1) * bl_box_pitch(bw) <= BL_BOX;
 }
