@@ -294,12 +294,11 @@ __global__ void k_awt_locate(const double *__restrict__ rel, int64_t nv, double 
 // the group holds; AW-towers groups hold a few visibilities (27 antennas x
 // 36 dumps at S = 128: 1.8).  The exponents are integers reduced mod M and
 // looked up in an FP64-rounded table, so the vectors carry FP32 rounding of
-// K terms only.  awtowers1800 (6991 groups, 12636 visibilities): 305 us in
+// K terms only.  awtowers1800 (6991 groups, 12636 visibilities): 289 us in
 // place of 6.1 ms (clear, pre-grid, transform and its copies, apply).  Bound
-// mainly by VALU issue: 130 million wave instructions, 212 us at 4 clocks on
-// 1024 SIMDs, against 3.9 million LDS and 5.5 million vector load ones.  So
-// Y read as two float4 instead of four float2 (306 us) and 8, 16 or 32 vectors
-// staged at a time (309, 305, 299 us) differ by 3 % at most.
+// mainly by VALU issue: 126 million wave instructions, 205 us at 4 clocks on
+// 1024 SIMDs, against 3.8 million LDS and 5.4 million vector load ones.  So
+// 8, 16 or 32 vectors staged at a time differ by 3 % at most.
 //
 // The vectors are centred, so the images carry the centring sign
 // (-1)^(x + y) that the pre-grids' uncentred transforms leave out (the input

@@ -386,10 +386,9 @@ __device__ __forceinline__ int wave_extreme(int v) {
 // values rounded to FP32 (kf, row pitch G).
 //
 // stream32k with 128 stations (66.6e6 visibilities, S = 8): one column per lane
-// from memory took 4.38 ms, pairs of columns (16-byte loads) 2.26 ms, bound by
-// L1 accesses (90 % of the cycles, ~18 per visibility, each row straddling
-// two 64-byte lines); from the LDS box 2.1
-// ms.
+// from memory took 4.38 ms, pairs of columns (16-byte loads) 2.26 ms, from the
+// LDS box 2.12 ms.  All 235 subgrids of 512 stations: 31.9 ms, 17.6 of them VALU
+// issue.
 typedef float bl_cell2 __attribute__((ext_vector_type(4), aligned(8)));  // two cells
 
 template <int G, int W>

@@ -183,11 +183,14 @@ __global__ __launch_bounds__(512) void k_wplane_sums(const double *__restrict__ 
 // the sum kept in FP64: the transformed planes never go back to memory.
 // Memory traffic is one read and one write of the stack for the rows and
 // one read for the columns, against four of each (two transposes), a copy
-// and k_wstack_add's read; that traffic is the bound.  Twiddles come from an
-// FP64-rounded table in LDS, so rounding matches a plain FP32 FFT.
+// and k_wstack_add's read.  Twiddles come from an FP64-rounded table in LDS, so
+// rounding matches a plain FP32 FFT.
 //
-// wstack2048 (65 planes): 960 + 1230 us, where the library transform, its
-// input copy and k_wstack_add took 4.67 ms.
+// wstack2048 (65 planes): 957 + 1384 us, where the library transform, its
+// input copy and k_wstack_add took 4.67 ms.  The rows are bound by that traffic
+// (4.56 TB/s, a large copy 4.79); the columns move 1.86 TB/s and issue VALU
+// instructions for 614 us, the rest exposed between the barriers of the one
+// workgroup per compute unit.
 template <int L>
 struct WstFft {
   static constexpr int N = 1 << L;
