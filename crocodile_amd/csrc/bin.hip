@@ -21,7 +21,11 @@ namespace {
 constexpr int BIN_NT = 1024;
 // Visibilities per thread of the counting and scattering passes: 8 amortise
 // the block histogram, 1 spreads small calls over the chip (1.3e5
-// visibilities: 16 blocks of 8192 took 28 us, 128 of 1024 8 us).
+// visibilities: 16 blocks of 8192 took 28 us, 128 of 1024 8 us), as long as a
+// compute unit gets one block (its histogram lets no second one in).  A whole
+// binning, 1 / 8 per thread: 130000 visibilities 48 / 69 us (N = 512), 80 / 103
+// (N = 2048, 100 planes), 79 / 104 (N = 8192); 260000 55 / 70, 91 / 107, 90 / 106;
+// 520000 68 / 73, 113 / 111, 116 / 113.
 constexpr int BIN_PER_MAX = 8;
 constexpr int HIST_MAX = 32768;  // 128 KiB of LDS
 template <int BIN_PER>
@@ -381,7 +385,7 @@ int bin_visibilities(croc_ctx *ctx, WsSet &set, const BinArgs &a, int max_suppor
   hipStream_t s = ctx->stream;
   if ((rc = zero2_u32_async(ctx, p.count, p.nbins + 1, small, 24))) return rc;
   const BinGeom g{T, p.ntx, p.ngroups, p.group_elems};
-  const bool spread = a.nv < (int64_t)BIN_NT * BIN_PER_MAX * ctx->num_cu / 4;
+  const bool spread = a.nv <= (int64_t)BIN_NT * ctx->num_cu;
   const int64_t vpb = spread ? BIN_NT : BIN_NT * BIN_PER_MAX;
   const int nblk = (int)((a.nv + vpb - 1) / vpb);
   if (nblk > 0) {
