@@ -868,6 +868,11 @@ bool box_inside(int N, int S, double theta, double du, double dv, double min_u, 
 // every selectable window lies inside its grid (box_inside), so only the
 // chunk ranges are validated and the degrid pass counts; otherwise a
 // per-visibility pass checks every window and counts.
+// Counts of the degrid pass up to which the host adds them up; more take a
+// launch of their own (120 baselines of 32 x 8 visibilities: 89 us a call, 120
+// with the launch).
+constexpr int64_t BL_HOST_COUNTS = 1024;
+
 int degrid_run(croc_ctx *ctx, DegridArgs a, bool safe, uint64_t *ndeg_total) {
   if (a.c.n == 0) {
     if (ndeg_total) *ndeg_total = 0;
@@ -917,7 +922,15 @@ int degrid_run(croc_ctx *ctx, DegridArgs a, bool safe, uint64_t *ndeg_total) {
   if ((rc = tap_timer_end(ctx, 1))) return rc;
   CROC_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
   ctx->ev_degrid = true;
-  if (ndeg_total) {
+  if (ndeg_total && safe && a.c.n <= BL_HOST_COUNTS) {
+    unsigned long long *h =
+        (unsigned long long *)host_stage(ctx, sizeof(unsigned long long) * BL_HOST_COUNTS);
+    if (!h) return CROC_ENOMEM;
+    CROC_HIP(hipMemcpyAsync(h, a.count, sizeof(*h) * a.c.n, hipMemcpyDeviceToHost, ctx->stream));
+    CROC_HIP(hipStreamSynchronize(ctx->stream));
+    *ndeg_total = 0;
+    for (int64_t k = 0; k < a.c.n; k++) *ndeg_total += h[k];
+  } else if (ndeg_total) {
     if (safe) {
       k_bl_total<<<1, 1024, 0, ctx->stream>>>(a.count, a.c.n, a.total);
       CROC_HIP(hipGetLastError());

@@ -431,3 +431,22 @@ def test_degrid_windows_across_a_large_grid(gpu):
     in_turn = BL.degrid_conv_uv(gd, N, theta, u.T.ravel(), v.T.ravel(), k).cpu().numpy()
     assert (by_corner != 0).all()
     assert_array_equal(in_turn.reshape(n, 4).T.ravel(), by_corner)
+
+
+@pytest.mark.parametrize('n', [1, 1024, 1025])
+def test_streamer_flops_by_chunks(gpu, n):
+    """The flop count is the counts' sum where the host adds them up (up to 1024
+    chunks) and where a launch does."""
+    print('case streamer flops n=%d' % n, flush=True)
+    rng = numpy.random.default_rng(n)
+    theta, S, Q, xM, xA, tc, fc = 0.05, 6, 32, 128, 64, 4, 4
+    _, sub = rand_grid(rng, xM)
+    host, dev = make_set(rng, 70, 16, 16, 2500.0, with_vis=False)
+    chunks = numpy.array([[b, t, t + tc, f, f + fc] for b in range(host.nbl)
+                          for t in range(0, 16, tc) for f in range(0, 16, fc)],
+                         dtype=numpy.int32)[:n]
+    box = (-xA / 2 / theta, xA / 2 / theta, -xA / 2 / theta, xA / 2 / theta)
+    _, nd, flops = BL.streamer_degrid_worker(dev, sub, xM, theta, 0.0, 0.0, chunks, *box,
+                                             BL.SepKernelData(rng.normal(size=(Q, S))), tc, fc)
+    assert len(nd) == n and (n == 1 or int(nd.sum()) > 0)
+    assert flops == int(nd.sum()) * 4 * (1 + S) * S
